@@ -17,7 +17,10 @@
 #include "fc_internal.h"
 #include "fc_vocab.h"
 
-#define EMBED_MAXW 1024
+#define EMBED_MAXW 1024       // tokens per row a chunk may hold
+// Chunks of at most this many tokens per row walk them in k_embed (one
+// launch, one workgroup per row); longer ones take k_embed_tok.
+#define EMBED_SERIAL_MAX 32
 
 // Eight consecutive entries of an embedding row as fp32.
 __device__ __forceinline__ void ld8(const bf16_t* p, float* o) {
@@ -60,7 +63,7 @@ __global__ __launch_bounds__(256) void k_embed(const T* __restrict__ wte, const 
                                                float* __restrict__ x0, int* __restrict__ tok_row,
                                                int* __restrict__ tok_pos, int full_smear, bf16_t* __restrict__ h,
                                                DraftMerge dm) {
-  __shared__ float sg[EMBED_MAXW], sinv[EMBED_MAXW];
+  __shared__ float sg[EMBED_SERIAL_MAX], sinv[EMBED_SERIAL_MAX];
   const int b = blockIdx.x;
   // NORM with dm.part: first finish the previous draft step for this row; its
   // draft is the row's one token here (written to tokens[] for the later
@@ -197,6 +200,193 @@ __global__ __launch_bounds__(256) void k_embed(const T* __restrict__ wte, const 
       }
     }
   }
+}
+
+// The embedding of longer chunks (prompts, whole sequences), one wave per
+// token. k_embed keeps a row in one workgroup, which leaves a batch of
+// prompts on as many CUs as it has rows: 277 us for 16 rows of up to 256
+// tokens (n_embd 1536, decode smear) and 1336 us for 4 x 1500 (n_embd 768,
+// full smear, two chunks), where these kernels take 37 and 26 us (latency-
+// bound: one read and three fp32 writes per element, 67 and 84 MB).
+//   full_smear: x_t = n_t + g_t n_{t-1} needs only the token before it, so
+//     the wave normalises both and writes everything.
+//   decode smear: x_t = n_t + g_t x_{t-1} is a chain; this kernel leaves each
+//     token's 1 / rms and gate in `ng` and k_embed_scan walks the chain.
+// Sums and arithmetic are those of k_embed, in its order.
+template <typename T>
+__global__ __launch_bounds__(256) void k_embed_tok(const T* __restrict__ wte, const float* __restrict__ smear_gate,
+                                                   float smear_lambda, float r0, float a0,
+                                                   const int* __restrict__ tokens, const int* __restrict__ row_off,
+                                                   const int* __restrict__ start, int max_per_row, int Mcap, int D,
+                                                   int cap, float* __restrict__ hist, float* __restrict__ x,
+                                                   float* __restrict__ x0, int* __restrict__ tok_row,
+                                                   int* __restrict__ tok_pos, int full_smear,
+                                                   float2* __restrict__ ng) {
+  const int b = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const RowSpan sp = row_span(row_off, b, max_per_row, Mcap);
+  const int base = sp.base, n = sp.n, s0 = start[b];
+  if (n <= 0 || s0 < 0) {  // a rejected row's packed slots get row -1 (see k_embed)
+    if (blockIdx.x != 0) return;
+    const int lo = max(row_off[b], 0), hi = min(row_off[b + 1], Mcap);
+    for (int j = lo + (int)threadIdx.x; j < hi; j += blockDim.x) tok_row[j] = -1;
+    return;
+  }
+  const int j = blockIdx.x * 4 + wave;
+  if (j >= n) return;
+  const int64_t m = base + j;
+  const int pos = s0 + j;
+  if (lane == 0) {
+    tok_row[m] = b;
+    tok_pos[m] = pos;
+  }
+  const T* e = wte + (int64_t)tokens[m] * D;
+  const T* pe = full_smear && j > 0 ? wte + (int64_t)tokens[m - 1] * D : nullptr;
+  float ss = 0.f, ps = 0.f;
+  for (int d = lane * 8; d < D; d += 64 * 8) {
+    float v[8];
+    ld8(e + d, v);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ss += v[i] * v[i];
+    if (pe != nullptr) {
+      ld8(pe + d, v);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) ps += v[i] * v[i];
+    }
+  }
+  ss = wave_sum(ss);
+  const float inv = 1.f / sqrtf(ss / (float)D + 1e-6f);
+  const float z = wave_sum(lane < 24 ? (ld<T>(e, lane) * inv) * smear_gate[lane] : 0.f);
+  const float g = smear_lambda * (1.f / (1.f + expf(-z)));
+  if (!full_smear) {
+    if (lane == 0) ng[m] = make_float2(inv, g);
+    return;
+  }
+  const float pinv = pe != nullptr ? 1.f / sqrtf(wave_sum(ps) / (float)D + 1e-6f) : 0.f;
+  for (int c0 = lane * 8; c0 < D; c0 += 64 * 8) {
+    float prev[8], nv[8], xv[8], xr[8];
+    if (pe != nullptr) {
+      ld8(pe + c0, prev);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) prev[i] *= pinv;
+    } else if (s0 > 0) {
+      ld8(hist + ((int64_t)b * cap + s0 - 1) * D + c0, prev);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) prev[i] = 0.f;
+    }
+    ld8(e + c0, nv);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      nv[i] *= inv;
+      xv[i] = nv[i] + g * prev[i];
+      xr[i] = r0 * xv[i] + a0 * xv[i];
+    }
+    if (pos < cap) st8(hist + ((int64_t)b * cap + pos) * D + c0, nv);
+    st8(x0 + m * D + c0, xv);
+    st8(x + m * D + c0, xr);
+  }
+}
+
+// The decode smear's chain after k_embed_tok: a workgroup owns 128 columns of
+// a row (12 workgroups per row at n_embd 1536). Its first wave walks the
+// chain, two columns per lane, EMBED_SCAN_BLK tokens at a time into LDS, its
+// only memory operations the embedding loads one block ahead; the other three
+// waves each write one of the outputs from the block before. (One wave doing
+// both took 41 us for 16 rows x 256 tokens: loads and stores retire in order,
+// at most 63 outstanding, so every load waited for the write acknowledgements
+// of the tokens before it. Here 31 us, the chain's own ~100 cycles per token.) Token ids, norms and gates of 64
+// tokens are held one per lane and broadcast from there, so that no index
+// load stands before an embedding load.
+#define EMBED_SCAN_BLK 32
+// two consecutive entries as loaded, and as fp32
+template <typename T> struct Raw2;
+template <> struct Raw2<bf16_t> { typedef uint32_t t; };
+template <> struct Raw2<float> { typedef float2 t; };
+__device__ __forceinline__ float2 f2_of(uint32_t w) {
+  return make_float2(__uint_as_float(w << 16), __uint_as_float(w & 0xffff0000u));
+}
+__device__ __forceinline__ float2 f2_of(float2 w) { return w; }
+__device__ __forceinline__ float lane_float(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+template <typename T>
+__global__ __launch_bounds__(256) void k_embed_scan(const T* __restrict__ wte, float r0, float a0,
+                                                    const int* __restrict__ tokens, const int* __restrict__ row_off,
+                                                    const int* __restrict__ start, int max_per_row, int Mcap, int D,
+                                                    int cap, float* __restrict__ hist, float* __restrict__ x,
+                                                    float* __restrict__ x0, const float2* __restrict__ ng) {
+  __shared__ __align__(16) float buf[2][EMBED_SCAN_BLK][128];
+  const int b = blockIdx.y, c0 = blockIdx.x * 128, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const RowSpan sp = row_span(row_off, b, max_per_row, Mcap);
+  const int base = sp.base, n = sp.n, s0 = start[b];
+  if (n <= 0 || s0 < 0) return;  // the whole workgroup
+  const int nblk = (n + EMBED_SCAN_BLK - 1) / EMBED_SCAN_BLK;
+  if (wave == 0) {
+    const int c = min(c0 + 2 * lane, D - 2);  // lanes past D walk column D - 2 again; nothing stores theirs
+    typedef typename Raw2<T>::t raw;
+    float2 prev = make_float2(0.f, 0.f);
+    if (s0 > 0) prev = *(const float2*)(hist + ((int64_t)b * cap + s0 - 1) * D + c);
+    // lane l < 32: token 32 blk + l of this block, l >= 32: of the next
+    int tk = tokens[base + min(lane, n - 1)];
+    float2 q = ng[base + min(lane, n - 1)];
+    raw ev[EMBED_SCAN_BLK];
+#pragma unroll
+    for (int u = 0; u < EMBED_SCAN_BLK; ++u)
+      ev[u] = *(const raw*)(wte + (int64_t)__builtin_amdgcn_readlane(tk, u) * D + c);
+    for (int blk = 0; blk < nblk; ++blk) {
+      const int nx = base + min((blk + 1) * EMBED_SCAN_BLK + lane, n - 1);  // the next block's two
+      const int tk2 = tokens[nx];
+      const float2 q2 = ng[nx];
+#pragma unroll
+      for (int u = 0; u < EMBED_SCAN_BLK; ++u) {
+        const float qi = lane_float(q.x, u), qg = lane_float(q.y, u);
+        const float2 e = f2_of(ev[u]);
+        const float2 nv = make_float2(e.x * qi, e.y * qi);
+        prev = make_float2(nv.x + qg * prev.x, nv.y + qg * prev.y);  // past the row's end: stored nowhere
+        ev[u] = *(const raw*)(wte + (int64_t)__builtin_amdgcn_readlane(tk, 32 + u) * D + c);
+        *(float2*)&buf[blk & 1][u][2 * lane] = prev;
+      }
+      tk = tk2;
+      q = q2;
+      __syncthreads();
+    }
+    return;
+  }
+  // lane: column group 4 (lane % 32), tokens lane / 32, + 2, ...
+  const int c4 = 4 * (lane & 31), c = c0 + c4;
+  for (int blk = 0; blk < nblk; ++blk) {
+    __syncthreads();  // block blk is in LDS; wave 0 goes on to the other buffer
+    if (c >= D) continue;
+    const int jn = min(EMBED_SCAN_BLK, n - blk * EMBED_SCAN_BLK);
+#pragma unroll 4
+    for (int u = lane >> 5; u < jn; u += 2) {
+      const float4 v = *(const float4*)&buf[blk & 1][u][c4];
+      const int j = blk * EMBED_SCAN_BLK + u;
+      const int64_t o = (int64_t)(base + j) * D + c;
+      if (wave == 1) {
+        if (s0 + j < cap) *(float4*)(hist + ((int64_t)b * cap + s0 + j) * D + c) = v;
+      } else if (wave == 2) {
+        *(float4*)(x0 + o) = v;
+      } else {
+        *(float4*)(x + o) = make_float4(r0 * v.x + a0 * v.x, r0 * v.y + a0 * v.y, r0 * v.z + a0 * v.z,
+                                        r0 * v.w + a0 * v.w);
+      }
+    }
+  }
+}
+
+template <typename T>
+static void launch_embed_long(const fc_model* m, const fc_cache* c, const fc_chunk* ch, int full_smear, float* x,
+                              float* x0, int* tok_row, int* tok_pos, float2* ng, hipStream_t s) {
+  const int D = m->n_embd;
+  const float r0 = m->layers[0].resid_lambda, a0 = m->layers[0].x0_lambda;
+  hipLaunchKernelGGL(k_embed_tok<T>, dim3((ch->max_per_row + 3) / 4, c->batch), dim3(256), 0, s, (const T*)m->wte,
+                     m->smear_gate, m->smear_lambda, r0, a0, ch->tokens, ch->row_off, ch->start, ch->max_per_row,
+                     ch->max_tokens, D, c->cap, c->hist, x, x0, tok_row, tok_pos, full_smear, ng);
+  if (!full_smear)
+    hipLaunchKernelGGL(k_embed_scan<T>, dim3((D + 127) / 128, c->batch), dim3(256), 0, s, (const T*)m->wte, r0, a0,
+                       ch->tokens, ch->row_off, ch->start, ch->max_per_row, ch->max_tokens, D, c->cap, c->hist, x, x0,
+                       ng);
 }
 
 // A residual-stream update left pending by a split-K GEMM: the S partial
@@ -425,6 +615,10 @@ int fc_forward_vp(const fc_model* m, const fc_cache* c, const fc_chunk* ch, void
                        m->smear_lambda, m->layers[0].resid_lambda, m->layers[0].x0_lambda, ch->tokens, ch->row_off,
                        ch->start, ch->max_per_row, Mcap, D, c->cap, c->hist, w.x, w.x0, w.tok_row, w.tok_pos,
                        full_smear, (bf16_t*)w.h, dmv);
+  else if (ch->max_per_row > EMBED_SERIAL_MAX && dt == FC_BF16)  // `qkv` is free here: two floats per token
+    launch_embed_long<bf16_t>(m, c, ch, full_smear, w.x, w.x0, w.tok_row, w.tok_pos, (float2*)w.qkv, s);
+  else if (ch->max_per_row > EMBED_SERIAL_MAX)
+    launch_embed_long<float>(m, c, ch, full_smear, w.x, w.x0, w.tok_row, w.tok_pos, (float2*)w.qkv, s);
   else if (dt == FC_BF16)
     hipLaunchKernelGGL((k_embed<bf16_t, false>), dim3(B), dim3(256), 0, s, (const bf16_t*)m->wte, m->smear_gate,
                        m->smear_lambda, m->layers[0].resid_lambda, m->layers[0].x0_lambda, ch->tokens, ch->row_off,
