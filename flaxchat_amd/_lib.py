@@ -67,7 +67,8 @@ class FcSpecState(Structure):
 
 EXPORTS = ["fc_last_error", "fc_version", "fc_forward_workspace_bytes", "fc_forward", "fc_gemm", "fc_pack_operand",
            "fc_attention_workspace_bytes", "fc_attention", "fc_attention_noalloc", "fc_attention_noalloc_max_bytes",
-           "fc_attn_prologue", "fc_attn_qkv_workspace_bytes", "fc_attn_qkv", "fc_row_stats", "fc_spec_workspace_bytes",
+           "fc_attn_prologue", "fc_attn_qkv_workspace_bytes", "fc_attn_qkv", "fc_row_stats", "fc_row_stats_fields",
+           "fc_spec_workspace_bytes",
            "fc_spec_round", "fc_spec_accept", "fc_spec_part_bytes", "fc_fast_sample", "fc_engine_sample",
            "fc_cross_entropy", "fc_read_probe", "fc_l2_read_probe", "fc_walk_probe", "fc_gemm_walk_probe",
            "fc_gemm_walk_probe_words", "fc_graph_begin", "fc_graph_end", "fc_graph_launch", "fc_graph_destroy"]
@@ -105,6 +106,8 @@ def _declare(L):
     L.fc_attention.restype = i32
     L.fc_row_stats.argtypes = [vp, i32, i32, f32, i32, vp, vp]
     L.fc_row_stats.restype = i32
+    L.fc_row_stats_fields.argtypes = [vp, i32, i32, f32, i32, vp, vp, vp, vp, vp, vp]
+    L.fc_row_stats_fields.restype = i32
     L.fc_spec_round.argtypes = [POINTER(FcModel), POINTER(FcCache), POINTER(FcModel), POINTER(FcCache),
                                 POINTER(FcSpecState), vp, i64, vp]
     L.fc_spec_round.restype = i32

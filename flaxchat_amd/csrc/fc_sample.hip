@@ -209,23 +209,285 @@ __device__ int block_draw(const float* __restrict__ zp, const fc_rowstat& sp, co
   return bi;
 }
 
+// ---------------------------------------------------------------------------
+// Row statistics with the row in registers: thread t of the row's workgroup
+// holds entries 4 (1024 q + t) .. +3, q < NQ (V <= 4096 NQ), so the row is
+// read from memory once, all loads in flight together; row_stats_block reads
+// it seven times with one scalar load in flight per thread. At top_k the
+// keep set is searched among the few entries at or above a lower bound of
+// the k-th largest key: the k-th largest of the threads' maxima (k entries
+// reach it), of which the upper 16 bits are enough. 65536 entries, top_k 40:
+// 30 us for 224 rows (one per CU: the read, 59 MB, is 12 us of it; 198 us
+// through row_stats_block), and one sampling step of 16 rows 17 us (149 us).
+// ---------------------------------------------------------------------------
+struct RegSmem {
+  float redv[NTHR / 64], reds[NTHR / 64];
+  int redi[NTHR / 64];
+  uint32_t tmax[NTHR];           // the threads' largest keys, then the candidates in rank order
+  uint64_t cand[NTHR + 8];       // candidates: key, then ~index (ordered by value, lower index first)
+  uint32_t bound, tau;
+  int ncand, tie_idx, more_eq;
+  int sidx[NTHR];                // candidates' indices in rank order
+};
+
+// block_argmax / block_sum for NTHR threads, the waves' results merged by
+// lanes instead of one after another.
+__device__ __forceinline__ void row_argmax(float& v, int& i, RegSmem& sm) {
+  const int lane = threadIdx.x & 63;
+  wave_argmax(v, i);
+  if (lane == 0) {
+    sm.redv[threadIdx.x >> 6] = v;
+    sm.redi[threadIdx.x >> 6] = i;
+  }
+  __syncthreads();
+  v = sm.redv[lane & 15];
+  i = sm.redi[lane & 15];
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) argmax_merge(v, i, __shfl_xor(v, o, WAVE), __shfl_xor(i, o, WAVE));
+}
+__device__ __forceinline__ float row_sum(float v, RegSmem& sm) {
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) sm.reds[threadIdx.x >> 6] = v;
+  __syncthreads();
+  v = sm.reds[threadIdx.x & 15];
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
+  return v;
+}
+
+template <int NQ>
+__device__ __forceinline__ void reg_load_row(const float* __restrict__ z, int V, bool vec, float (&v)[NQ][4]) {
+  if (vec) {  // 16-byte aligned row, V % 4 == 0: whole groups
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const int e = 4 * (NTHR * q + (int)threadIdx.x);
+      float4 t = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      if (e < V) t = *(const float4*)(z + e);
+      v[q][0] = t.x; v[q][1] = t.y; v[q][2] = t.z; v[q][3] = t.w;
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const int e = 4 * (NTHR * q + (int)threadIdx.x);
+#pragma unroll
+      for (int w = 0; w < 4; ++w) v[q][w] = e + w < V ? z[e + w] : -INFINITY;
+    }
+  }
+}
+
+// The kk-th largest of the 64 N values mono(float) >> 16 held N per lane by
+// one wave (`n` of them real, in (u, lane) order; kk <= n): binary search
+// counted with ballots.
+template <int N>
+__device__ __forceinline__ uint32_t kth_top16(const uint32_t* __restrict__ key, int n, int kk) {
+  const int lane = threadIdx.x & 63;
+  uint32_t k[N];
+#pragma unroll
+  for (int u = 0; u < N; ++u) k[u] = lane + 64 * u < n ? key[lane + 64 * u] >> 16 : 0u;
+  uint32_t lo = 0u, hi = 0xffffu;
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi + 1u) >> 1;  // >= 1: absent values never count
+    int c = 0;
+#pragma unroll
+    for (int u = 0; u < N; ++u) c += wave_count(k[u] >= mid);
+    if (c >= kk) lo = mid;
+    else hi = mid - 1u;
+  }
+  return lo;
+}
+
+// row_stats_block's result from the row's registers. False (uniform over the
+// block, nothing returned) for rows it leaves to row_stats_block: one with a
+// NaN, and with top-k one whose bound is not a number (top_k threads without
+// a finite entry) or is reached by more than NTHR entries (equal values).
+// With top-k, sm.tmax / sm.sidx[0 .. top_k) then hold the kept keys and their
+// indices in rank order.
+template <int NQ>
+__device__ bool reg_row_stats(const float (&v)[NQ][4], int V, float T, int top_k, fc_rowstat& r, RegSmem& sm) {
+  const int tid = threadIdx.x, wave = tid >> 6;
+  // entries past V are -inf and never exceed anything
+  float bv = -INFINITY;
+  int bj = 0;
+  bool nan = false;
+#pragma unroll
+  for (int q = 0; q < NQ; ++q)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const bool up = v[q][w] > bv;
+      bv = up ? v[q][w] : bv;
+      bj = up ? 4 * q + w : bj;
+      nan |= v[q][w] != v[q][w];
+    }
+  int bi = 4 * (NTHR * (bj >> 2) + tid) + (bj & 3);
+  const bool filter = T > 0.f && top_k > 0 && top_k < V;
+  // the k-th largest of groups of 4 threads' maxima bounds a small k as well
+  // as the threads' own do, in a quarter of the counting
+  const bool coarse = top_k <= NTHR / 8;
+  if (tid == 0) sm.ncand = 0;
+  if (filter) {
+    float gm = bv;
+    if (coarse) {
+      gm = fmaxf(gm, __shfl_xor(gm, 1, WAVE));
+      gm = fmaxf(gm, __shfl_xor(gm, 2, WAVE));
+      if ((tid & 3) == 0) sm.tmax[tid >> 2] = mono(gm);
+    } else {
+      sm.tmax[tid] = mono(gm);
+    }
+  }
+  if (__syncthreads_or(nan)) return false;
+  if (filter && wave == 0) {
+    const int n = coarse ? min(NTHR / 4, (V + 15) / 16) : min(NTHR, (V + 3) / 4);
+    uint32_t lo = 0u;
+    if (top_k <= n) lo = coarse ? kth_top16<NTHR / 256>(sm.tmax, n, top_k) : kth_top16<NTHR / 64>(sm.tmax, n, top_k);
+    if (tid == 0) sm.bound = lo << 16;
+  }
+  row_argmax(bv, bi, sm);
+  r = fc_rowstat{};
+  r.argmax = bv == -INFINITY ? 0 : bi;
+  r.tie_idx = V;
+  r.tau = -INFINITY;
+  r.mx = 0.f;
+  r.sum = 1.f;
+  if (!(T > 0.f)) return true;
+  const float mx = bv / T;  // the largest z / T (z / T is monotone)
+  float s = 0.f;
+  if (filter) {
+    const uint32_t bound = sm.bound;
+    if (bound < 0x00800000u) return false;
+    const float bf = unmono(bound);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+      if (fmaxf(fmaxf(v[q][0], v[q][1]), fmaxf(v[q][2], v[q][3])) >= bf) {
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+          if (v[q][w] >= bf) {
+            const int p = atomicAdd(&sm.ncand, 1);
+            if (p < NTHR)
+              sm.cand[p] = (uint64_t)mono(v[q][w]) << 32 | (uint32_t)~(4 * (NTHR * q + tid) + w);
+          }
+      }
+    __syncthreads();
+    const int C = sm.ncand;
+    if (C > NTHR) return false;
+    if (tid < 8) sm.cand[C + tid] = 0ull;  // the count below goes in groups of 8
+    __syncthreads();
+    // rank among the candidates: larger key first, lower index among equals
+    int rank = NTHR;
+    uint32_t key = 0u;
+    if (tid < C) {
+      const uint64_t mine = sm.cand[tid];
+      key = (uint32_t)(mine >> 32);
+      const int idx = (int)~(uint32_t)mine;
+      rank = 0;
+      for (int i = 0; i < C; i += 8) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) rank += sm.cand[i + u] > mine;
+      }
+      sm.tmax[rank] = key;
+      sm.sidx[rank] = idx;
+      if (rank == top_k - 1) {
+        sm.tau = key;
+        sm.tie_idx = idx;
+        sm.more_eq = 0;
+      }
+    }
+    __syncthreads();
+    const uint32_t tau = sm.tau;
+    if (tid < C && rank >= top_k && key == tau) sm.more_eq = 1;  // equal entries that are not kept
+    if (tid < top_k) s = expf(unmono(sm.tmax[tid]) / T - mx);    // top_k <= C; rank order: a fixed sum
+    s = row_sum(s, sm);
+    r.tau = unmono(tau);
+    r.tie_idx = sm.more_eq ? sm.tie_idx : V;
+  } else {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float x = expf(v[q][w] / T - mx);
+        s += 4 * (NTHR * q + tid) + w < V ? x : 0.f;
+      }
+    s = row_sum(s, sm);
+  }
+  r.mx = mx;
+  r.sum = s;
+  return true;
+}
+
+// where a row's statistics go: an fc_rowstat, or one array per field
+struct StatOut {
+  fc_rowstat* rows;
+  float *mx, *sum, *tau;
+  int *tie_idx, *argmax;
+};
+__device__ __forceinline__ void put_stat(const StatOut& o, int row, const fc_rowstat& r) {
+  if (o.rows != nullptr) {
+    o.rows[row] = r;
+    return;
+  }
+  o.mx[row] = r.mx;
+  o.sum[row] = r.sum;
+  o.tau[row] = r.tau;
+  o.tie_idx[row] = r.tie_idx;
+  o.argmax[row] = r.argmax;
+}
+
+// NQ = 0: rows longer than 65536 entries (read from memory in every step).
+template <int NQ>
 __global__ __launch_bounds__(NTHR) void k_row_stats(const float* __restrict__ logits, int V, float T, int top_k,
-                                                    fc_rowstat* __restrict__ stats) {
+                                                    int vec, StatOut out) {
+  const float* z = logits + (int64_t)blockIdx.x * V;
+  if constexpr (NQ > 0) {
+    __shared__ RegSmem rs;
+    float v[NQ][4];
+    fc_rowstat r;
+    reg_load_row<NQ>(z, V, vec != 0, v);
+    if (reg_row_stats<NQ>(v, V, T, top_k, r, rs)) {
+      if (threadIdx.x == 0) put_stat(out, blockIdx.x, r);
+      return;
+    }
+  }
   __shared__ StatSmem sm;
-  row_stats_block(logits + (int64_t)blockIdx.x * V, V, T, top_k, stats + blockIdx.x, sm);
+  row_stats_block(z, V, T, top_k, nullptr, sm);
+  if (threadIdx.x == 0) put_stat(out, blockIdx.x, sm.res);
+}
+
+// groups of four entries per thread that hold a row of V entries (0: too long)
+static int reg_nq(int V) { return V <= 4 * NTHR * 4 ? 4 : V <= 4 * NTHR * 8 ? 8 : V <= 4 * NTHR * 16 ? 16 : 0; }
+static int rows_vec(const float* z, int V) { return V % 4 == 0 && (uintptr_t)z % 16 == 0; }
+
+static int launch_row_stats(const float* logits, int rows, int V, float T, int top_k, const StatOut& o, hipStream_t s) {
+  if (rows <= 0) return FC_OK;
+  const int vec = rows_vec(logits, V);
+#define ROW_STATS(NQ) hipLaunchKernelGGL(k_row_stats<NQ>, dim3(rows), dim3(NTHR), 0, s, logits, V, T, top_k, vec, o)
+  switch (reg_nq(V)) {
+    case 4: ROW_STATS(4); break;
+    case 8: ROW_STATS(8); break;
+    case 16: ROW_STATS(16); break;
+    default: ROW_STATS(0); break;
+  }
+#undef ROW_STATS
+  FC_LAUNCH_CHECK();
+  return FC_OK;
 }
 
 int fc_launch_row_stats(const float* logits, int rows, int V, float T, int top_k, fc_rowstat* stats, hipStream_t s) {
-  if (rows <= 0) return FC_OK;
-  hipLaunchKernelGGL(k_row_stats, dim3(rows), dim3(NTHR), 0, s, logits, V, T, top_k, stats);
-  FC_LAUNCH_CHECK();
-  return FC_OK;
+  StatOut o{};
+  o.rows = stats;
+  return launch_row_stats(logits, rows, V, T, top_k, o, s);
 }
 
 extern "C" int32_t fc_row_stats(const float* logits, int32_t rows, int32_t V, float temperature, int32_t top_k,
                                 fc_rowstat* stats, void* stream) {
   FC_CHECK_ARG(logits && stats && V > 0, "arguments");
   return fc_launch_row_stats(logits, rows, V, temperature, top_k, stats, (hipStream_t)stream);
+}
+
+extern "C" int32_t fc_row_stats_fields(const float* logits, int32_t rows, int32_t V, float temperature,
+                                       int32_t top_k, float* mx, float* sum, float* tau, int32_t* tie_idx,
+                                       int32_t* argmax, void* stream) {
+  FC_CHECK_ARG(logits && mx && sum && tau && tie_idx && argmax && V > 0, "arguments");
+  const StatOut o{nullptr, mx, sum, tau, tie_idx, argmax};
+  return launch_row_stats(logits, rows, V, temperature, top_k, o, (hipStream_t)stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -1406,15 +1668,17 @@ extern "C" int32_t fc_spec_round(const fc_model* target, const fc_cache* tcache,
 // ENGINE = false: rows stop on eos or at max_pos (done[] / max_pos[]).
 // ENGINE = true: no stop (completion is decided by the caller); a row with
 // forced[b] >= 0 takes that token instead of a sample.
-template <bool ENGINE>
+// NQ: the row in registers (reg_row_stats), 0 for rows longer than 65536.
+template <bool ENGINE, int NQ>
 __global__ __launch_bounds__(NTHR) void k_fast_sample(const float* __restrict__ logits, int V, float T, int top_k,
-                                                      uint64_t seed, int eos, int* __restrict__ gen, int gen_cap,
-                                                      int* __restrict__ pos, int* __restrict__ done,
+                                                      int vec, uint64_t seed, int eos, int* __restrict__ gen,
+                                                      int gen_cap, int* __restrict__ pos, int* __restrict__ done,
                                                       int* __restrict__ step, const int* __restrict__ max_pos,
                                                       const int* __restrict__ forced, int* __restrict__ tok_cur,
                                                       fc_rowstat* __restrict__ stats) {
-  __shared__ StatSmem sm;
-  const int b = blockIdx.x;
+  __shared__ float redv[16];
+  __shared__ int redi[16];
+  const int b = blockIdx.x, tid = threadIdx.x;
   int tok = -1;
   if (ENGINE) {
     tok = forced[b];
@@ -1423,32 +1687,68 @@ __global__ __launch_bounds__(NTHR) void k_fast_sample(const float* __restrict__ 
   }
   if (tok < 0) {
     const float* z = logits + (int64_t)b * V;
-    row_stats_block(z, V, T, top_k, stats + b, sm);
-    const fc_rowstat rs = sm.res;
-    if (T > 0.f) {
-      const uint32_t tk = mono(rs.tau);
-      const int rnd = step[b];
-      float bv = -INFINITY;
-      int bi = 0x7fffffff;
-      const int ngrp = (V + 3) >> 2;
-      for (int gi = threadIdx.x; gi < ngrp; gi += NTHR) {
-        const u32x4 r = philox4x32_10(u32x4{(uint32_t)gi, (uint32_t)b, (uint32_t)rnd, 0u}, (uint32_t)seed,
-                                      (uint32_t)(seed >> 32));
+    const int rnd = step[b];
+    float bv = -INFINITY;
+    int bi = 0x7fffffff;
+    auto noise = [&](int gi) {
+      return philox4x32_10(u32x4{(uint32_t)gi, (uint32_t)b, (uint32_t)rnd, 0u}, (uint32_t)seed,
+                           (uint32_t)(seed >> 32));
+    };
+    fc_rowstat rs;
+    bool reg = false;
+    if constexpr (NQ > 0) {
+      __shared__ RegSmem rsm;
+      float v[NQ][4];
+      reg_load_row<NQ>(z, V, vec != 0, v);
+      reg = reg_row_stats<NQ>(v, V, T, top_k, rs, rsm);
+      if (reg && tid == 0) stats[b] = rs;
+      if (reg && T > 0.f) {
+        if (top_k > 0 && top_k < V) {  // the keep set in rank order, one entry per thread
+          if (tid < top_k) {
+            const int i = rsm.sidx[tid];
+            argmax_merge(bv, bi, unmono(rsm.tmax[tid]) / T + gumbel_of(pick(noise(i >> 2), i & 3)), i);
+          }
+        } else {
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          const int i = gi * 4 + w;
-          if (i >= V) break;
-          if (!kept(z[i], i, tk, rs.tie_idx)) continue;
-          argmax_merge(bv, bi, z[i] / T + gumbel_of(pick(r, w)), i);
+          for (int q = 0; q < NQ; ++q) {
+            const int gi = NTHR * q + tid;
+            if (4 * gi < V) {
+              const u32x4 r = noise(gi);
+#pragma unroll
+              for (int w = 0; w < 4; ++w)
+                if (4 * gi + w < V) argmax_merge(bv, bi, v[q][w] / T + gumbel_of(pick(r, w)), 4 * gi + w);
+            }
+          }
         }
       }
-      block_argmax(bv, bi, sm.redv, sm.redi);
+    }
+    if (!reg) {
+      __shared__ StatSmem sm;
+      row_stats_block(z, V, T, top_k, stats + b, sm);
+      rs = sm.res;
+      if (T > 0.f) {
+        const uint32_t tk = mono(rs.tau);
+        const int ngrp = (V + 3) >> 2;
+        for (int gi = tid; gi < ngrp; gi += NTHR) {
+          const u32x4 r = noise(gi);
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            const int i = gi * 4 + w;
+            if (i >= V) break;
+            if (!kept(z[i], i, tk, rs.tie_idx)) continue;
+            argmax_merge(bv, bi, z[i] / T + gumbel_of(pick(r, w)), i);
+          }
+        }
+      }
+    }
+    if (T > 0.f) {
+      block_argmax(bv, bi, redv, redi);
       tok = bi;
     } else {
       tok = rs.argmax;
     }
   }
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     const int p = pos[b] + 1;
     if (p < gen_cap) gen[(int64_t)b * gen_cap + p] = tok;
     pos[b] = p;
@@ -1458,16 +1758,33 @@ __global__ __launch_bounds__(NTHR) void k_fast_sample(const float* __restrict__ 
   }
 }
 
+template <bool ENGINE>
+static int launch_fast_sample(const float* logits, int batch, int V, float T, int top_k, uint64_t seed, int eos,
+                              int* gen, int gen_cap, int* pos, int* done, int* step, const int* max_pos,
+                              const int* forced, int* tok_cur, fc_rowstat* stats, hipStream_t s) {
+  const int vec = rows_vec(logits, V);
+#define FAST_SAMPLE(NQ)                                                                                         \
+  hipLaunchKernelGGL((k_fast_sample<ENGINE, NQ>), dim3(batch), dim3(NTHR), 0, s, logits, V, T, top_k, vec, seed, \
+                     eos, gen, gen_cap, pos, done, step, max_pos, forced, tok_cur, stats)
+  switch (reg_nq(V)) {
+    case 4: FAST_SAMPLE(4); break;
+    case 8: FAST_SAMPLE(8); break;
+    case 16: FAST_SAMPLE(16); break;
+    default: FAST_SAMPLE(0); break;
+  }
+#undef FAST_SAMPLE
+  FC_LAUNCH_CHECK();
+  return FC_OK;
+}
+
 extern "C" int32_t fc_fast_sample(const float* logits, int32_t batch, int32_t V, float temperature, int32_t top_k,
                                   uint64_t seed, int32_t eos, int32_t* gen, int32_t gen_cap, int32_t* pos,
                                   int32_t* done, int32_t* step, const int32_t* max_pos, int32_t* tok_cur,
                                   fc_rowstat* stats, void* stream) {
   FC_CHECK_ARG(logits && gen && pos && done && step && max_pos && tok_cur && stats, "null pointer");
   FC_CHECK_ARG(batch > 0 && V > 0 && gen_cap > 0, "sizes");
-  hipLaunchKernelGGL(k_fast_sample<false>, dim3(batch), dim3(NTHR), 0, (hipStream_t)stream, logits, V, temperature,
-                     top_k, seed, eos, gen, gen_cap, pos, done, step, max_pos, nullptr, tok_cur, stats);
-  FC_LAUNCH_CHECK();
-  return FC_OK;
+  return launch_fast_sample<false>(logits, batch, V, temperature, top_k, seed, eos, gen, gen_cap, pos, done, step,
+                                   max_pos, nullptr, tok_cur, stats, (hipStream_t)stream);
 }
 
 extern "C" int32_t fc_engine_sample(const float* logits, int32_t batch, int32_t V, float temperature, int32_t top_k,
@@ -1475,10 +1792,8 @@ extern "C" int32_t fc_engine_sample(const float* logits, int32_t batch, int32_t 
                                     int32_t* step, int32_t* tok_cur, fc_rowstat* stats, void* stream) {
   FC_CHECK_ARG(logits && forced && gen && pos && step && tok_cur && stats, "null pointer");
   FC_CHECK_ARG(batch > 0 && V > 0 && gen_cap > 0, "sizes");
-  hipLaunchKernelGGL(k_fast_sample<true>, dim3(batch), dim3(NTHR), 0, (hipStream_t)stream, logits, V, temperature,
-                     top_k, seed, -1, gen, gen_cap, pos, nullptr, step, nullptr, forced, tok_cur, stats);
-  FC_LAUNCH_CHECK();
-  return FC_OK;
+  return launch_fast_sample<true>(logits, batch, V, temperature, top_k, seed, -1, gen, gen_cap, pos, nullptr, step,
+                                  nullptr, forced, tok_cur, stats, (hipStream_t)stream);
 }
 
 // ---------------------------------------------------------------------------

@@ -350,11 +350,11 @@ def row_stats(logits: torch.Tensor, temperature: float, top_k: int) -> Tuple[tor
     if logits.dtype != torch.float32 or logits.dim() != 2 or not logits.is_contiguous():
         raise ValueError("row_stats takes contiguous fp32 logits [rows][V]")
     rows, V = logits.shape
-    raw = torch.empty((rows, 8), dtype=torch.int32, device=logits.device)
-    check(lib().fc_row_stats(logits.data_ptr(), rows, V, temperature, top_k, raw.data_ptr(), _stream(logits)),
-          "fc_row_stats")
-    f = raw.view(torch.float32)
-    return f[:, 0].clone(), f[:, 1].clone(), f[:, 2].clone(), raw[:, 3].clone(), raw[:, 4].clone()
+    f = [torch.empty(rows, dtype=torch.float32, device=logits.device) for _ in range(3)]
+    i = [torch.empty(rows, dtype=torch.int32, device=logits.device) for _ in range(2)]
+    check(lib().fc_row_stats_fields(logits.data_ptr(), rows, V, temperature, top_k, *[t.data_ptr() for t in f + i],
+                                    _stream(logits)), "fc_row_stats_fields")
+    return f[0], f[1], f[2], i[0], i[1]
 
 
 @row_stats.register_fake

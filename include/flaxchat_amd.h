@@ -268,6 +268,10 @@ int32_t fc_attn_qkv(const fc_model* m, int32_t layer, const fc_cache* c, const v
 int32_t fc_row_stats(const float* logits, int32_t rows, int32_t V, float temperature,
                      int32_t top_k, fc_rowstat* stats, void* stream);
 
+/* fc_row_stats with one array of `rows` entries per field instead of fc_rowstat records. */
+int32_t fc_row_stats_fields(const float* logits, int32_t rows, int32_t V, float temperature, int32_t top_k,
+                            float* mx, float* sum, float* tau, int32_t* tie_idx, int32_t* argmax, void* stream);
+
 /* One speculative round on device (flaxchat/engine.py:484-606 with the
  * sequential verify replaced by one (pending + k)-token verify chunk and the
  * re-prefill replaced by length-pointer rollback): draft k steps, verify,
