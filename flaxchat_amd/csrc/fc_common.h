@@ -23,6 +23,29 @@ __device__ __forceinline__ f32x16 mfma32(v4u a, v4u b, f32x16 c) {
 
 #define WAVE 64
 
+// Direct global-to-LDS load of 1 KB by a wave: lane l's 16 bytes from
+// base + off (off = 16 l for a contiguous block) to LDS byte address
+// lds + 16 l. base and lds are uniform over the wave. The kernels that use it
+// wait for it themselves (vmcnt, then a barrier) before they read the LDS.
+// It is written in assembly, not with the builtin, for the sake of those
+// reads: the compiler tracks the builtin's LDS writes, loses track of which
+// object each went to where control flow merges (the head of every K loop),
+// and waits there for all loads in flight (vmcnt(0)) before the first LDS
+// read, which drained the ring of every kernel here once per loop iteration
+// (128 x 128 tiles, K 6144: 69 us with the builtin, 37 us with this). M0 has
+// to be written at least one cycle ahead of the load.
+template <bool NT = false>
+__device__ __forceinline__ void lds_load_1k(const void* base, uint32_t off, uint32_t lds) {
+  if constexpr (NT)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(base), "s"(lds)
+                 : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
+                 : "memory", "m0");
+}
+// LDS byte address of a __shared__ object
+#define LDS_ADDR(obj) ((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)&(obj))
+
 __device__ __forceinline__ float bf2f(bf16_t h) { return __uint_as_float(((uint32_t)h) << 16); }
 __device__ __forceinline__ bf16_t f2bf(float f) {
   // round to nearest even (inputs here are finite)

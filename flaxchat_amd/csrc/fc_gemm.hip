@@ -20,9 +20,9 @@
 //              into a 4-stage ring; verify c_fc.
 //   k_gemm_ring bf16 MFMA, 64 x 96 tiles, a 5-stage direct-load LDS ring;
 //              the verify MLP c_proj (K split 4).
-//   k_gemm_big bf16 MFMA, 256 x 256 tiles, 4-stage LDS ring of direct
-//              loads; prefill chunks (M >= 1024) and the lm_head from 200
-//              rows (the verify head).
+//   k_gemm_big bf16 MFMA, 128 x 128 to 256 x 256 tiles, 4-stage LDS ring of
+//              direct loads; prompt and whole-sequence chunks, large-batch
+//              verify chunks, and the lm_head from 200 rows.
 // The row count may be a device value (packed token chunks whose size is
 // only known on the GPU): the grid covers the capacity and tiles past the
 // actual count exit at once.
@@ -205,12 +205,10 @@ __global__ __launch_bounds__(256) void k_gemv(const T* __restrict__ A, const T* 
 // The same for the lm_head on the K-split kernel (one-row decode: cfg2's
 // 100 MB head read five times a round; 0.917-0.918 vs 0.924 ms per round)
 // and on the 256 x 256 kernel's direct loads (the cfg4 verify head:
-// 4.835-4.837 vs 4.840-4.845 ms per round), alternating builds.
+// 4.835-4.837 vs 4.840-4.845 ms per round; with more than one M tile the
+// tiles share the weights through the caches instead), alternating builds.
 #ifndef FC_KS_LM_NT
 #define FC_KS_LM_NT 1
-#endif
-#ifndef FC_BIG_LM_NT
-#define FC_BIG_LM_NT 1
 #endif
 __device__ __forceinline__ f32x4 mfma16(uint4 a, uint4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
@@ -978,16 +976,16 @@ __global__ __launch_bounds__(256) void k_gemm_dma(const bf16_t* __restrict__ A, 
   const int m0 = mt * 16 * MB;
   if (m0 >= M) return;
   const int n0 = nt * 64 * NBW;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t KS32 = K >> 5;
   const int C = K >> 6;
   const int last_blk = (M - 1) >> 4;
-  const bf16_t* wbase = W + ((int64_t)(n0 / 16 + wave * NBW)) * KS32 * 512 + lane * 8;
+  const bf16_t* wbase = W + ((int64_t)(n0 / 16 + wave * NBW)) * KS32 * 512;
   const bf16_t* abase[AB / WAVES];
 #pragma unroll
   for (int u = 0; u < AB / WAVES; ++u) {
     const int q = wave + WAVES * u;  // row block q / 2, k step q % 2
-    abase[u] = A + ((int64_t)min(m0 / 16 + (q >> 1), last_blk) * KS32 + (q & 1)) * 512 + lane * 8;
+    abase[u] = A + ((int64_t)min(m0 / 16 + (q >> 1), last_blk) * KS32 + (q & 1)) * 512;
   }
   RmsPre rpre;  // folded RMSNorm: this thread's share of row m0 + t / (256 / MT)
   if constexpr (EPI == EPI_RELU2) {
@@ -1003,16 +1001,16 @@ __global__ __launch_bounds__(256) void k_gemm_dma(const bf16_t* __restrict__ A, 
   constexpr int PER = 2 * NBW + AB / WAVES;
   constexpr int NV = PER * (NSTG - 2);
   static_assert(NV < 64, "vmcnt range");
+  const uint32_t voff = lane * 16;
 #define DMA_ISSUE(S, c_)                                                                             \
   {                                                                                                  \
     const int c = min((c_), C - 1); /* past the end: harmless re-reads into an unread stage */       \
+    const uint32_t lw_ = LDS_ADDR(S.w[0]) + 2048 * NBW * wave, la_ = LDS_ADDR(S.a[0]) + 1024 * wave; \
     _Pragma("unroll") for (int j = 0; j < NBW; ++j)                                                  \
       _Pragma("unroll") for (int ks = 0; ks < 2; ++ks)                                               \
-        __builtin_amdgcn_global_load_lds((const void*)(wbase + ((int64_t)j * KS32 + 2 * c + ks) * 512), \
-                                         (__attribute__((address_space(3))) void*)&S.w[wave][2 * j + ks][0], 16, 0, 0); \
+        lds_load_1k(wbase + ((int64_t)j * KS32 + 2 * c + ks) * 512, voff, lw_ + 1024 * (2 * j + ks)); \
     _Pragma("unroll") for (int u = 0; u < AB / WAVES; ++u)                                           \
-      __builtin_amdgcn_global_load_lds((const void*)(abase[u] + (int64_t)c * 1024),                  \
-                                       (__attribute__((address_space(3))) void*)&S.a[wave + WAVES * u][0], 16, 0, 0); \
+      lds_load_1k(abase[u] + (int64_t)c * 1024, voff, la_ + 1024 * WAVES * u);                       \
   }
 #define DMA_STEP(S, SN, i_)                                                                          \
   {                                                                                                  \
@@ -1102,7 +1100,7 @@ __global__ __launch_bounds__(256) void k_gemm_ring(const bf16_t* __restrict__ A,
   const int m0 = mt * 16 * MB;
   if (m0 >= M) return;
   const int n0 = nt * 16 * NB;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave / WN, wn = wave % WN;
   const int r = lane & 15, g = lane >> 4;
   const int C = K >> 6;
@@ -1121,10 +1119,10 @@ __global__ __launch_bounds__(256) void k_gemm_ring(const bf16_t* __restrict__ A,
     const int q = min(wave + 4 * u, TOT - 1);
     dst[u] = q;
     if (q < 2 * MB) {
-      src[u] = A + ((int64_t)min(m0 / 16 + (q >> 1), last_blk) * KS32 + (q & 1)) * 512 + lane * 8;
+      src[u] = A + ((int64_t)min(m0 / 16 + (q >> 1), last_blk) * KS32 + (q & 1)) * 512;
     } else {
       const int j2 = q - 2 * MB;
-      src[u] = W + ((int64_t)(n0 / 16 + (j2 >> 1)) * KS32 + (j2 & 1)) * 512 + lane * 8;
+      src[u] = W + ((int64_t)(n0 / 16 + (j2 >> 1)) * KS32 + (j2 & 1)) * 512;
     }
   }
   RmsPre rpre;  // folded RMSNorm: this thread's share of row m0 + t / (256 / MT)
@@ -1136,14 +1134,13 @@ __global__ __launch_bounds__(256) void k_gemm_ring(const bf16_t* __restrict__ A,
   for (int i = 0; i < MBW; ++i)
 #pragma unroll
     for (int j = 0; j < NBW; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint32_t voff = lane * 16;
 #define RING_STG(k) (k == 0 ? s0 : k == 1 ? s1 : k == 2 ? s2 : k == 3 ? s3 : k == 4 ? s4 : k == 5 ? s5 : k == 6 ? s6 : s7)
 #define RING_ISSUE(k, c_)                                                                                  \
   {                                                                                                        \
     const int64_t cc_ = (int64_t)(c_beg + min((c_), n - 1)) * 1024; /* past the end: harmless re-reads */  \
-    _Pragma("unroll") for (int u = 0; u < PER; ++u)                                                        \
-      __builtin_amdgcn_global_load_lds((const void*)(src[u] + cc_),                                        \
-                                       (__attribute__((address_space(3))) void*)&RING_STG(k).blk[dst[u]][0], \
-                                       16, 0, 0);                                                          \
+    const uint32_t l_ = LDS_ADDR(RING_STG(k).blk[0]);                                                      \
+    _Pragma("unroll") for (int u = 0; u < PER; ++u) lds_load_1k(src[u] + cc_, voff, l_ + 1024 * dst[u]);   \
   }
 #define RING_STEP(k, i_)                                                                                   \
   {                                                                                                        \
@@ -1226,36 +1223,45 @@ __global__ __launch_bounds__(256) void k_gemm_ring(const bf16_t* __restrict__ A,
   }
 }
 
-// bf16 MFMA GEMM for prefill-size row counts (M >= FC_BIG_M, N % 256 == 0,
-// K % 128 == 0).
+// bf16 MFMA GEMM for prompt and whole-sequence row counts.
 //
-// A workgroup owns a 256 x 256 output tile; each of its four waves owns a
-// 128 x 128 quadrant as 4 x 4 blocks of 32 x 32 (the 32x32x16 MFMA: with
-// one wave per SIMD it keeps the matrix unit ~86% busy, where 16x16x32
-// chains reach about half), 256 accumulators per lane. Per 32-wide k step
-// the tile needs 16 activation and 16 weight blocks of 1 KB (16 rows x 32 k,
-// fragment order); they go straight from global memory into one of four
-// 32 KB LDS stages by direct loads, 8 per wave. The 32x32x16 operand of
-// lane l is row l % 32, k 8 (l / 32) .. +7 of a 16-k half: 16 bytes that sit
-// in 16-row block (l % 32) / 16 at lane slot l % 16 + 16 (2 half + l / 32),
-// so the stored layout feeds it unchanged.
+// A workgroup owns a 64 MB x 64 NB output tile; each of its 2 x 2 waves owns
+// MB x NB blocks of 32 x 32 (the 32x32x16 MFMA: with one wave per SIMD it
+// keeps the matrix unit ~86% busy, where 16x16x32 chains reach about half).
+// Per 32-wide k step the tile needs 4 MB activation and 4 NB weight blocks of
+// 1 KB (16 rows x 32 k, fragment order); they go straight from global memory
+// into one of four LDS stages by direct loads, MB + NB per wave. The
+// 32x32x16 operand of lane l is row l % 32, k 8 (l / 32) .. +7 of a 16-k half:
+// 16 bytes that sit in 16-row block (l % 32) / 16 at lane slot
+// l % 16 + 16 (2 half + l / 32), so the stored layout feeds it unchanged.
 //
-// Per step i: wait until stage i+1 has landed (own loads: vmcnt(16), the two
+// Per step i: wait until stage i+1 has landed (own loads: vmcnt, the two
 // later stages may still be in flight) and every wave has finished reading
 // stage i into registers (lgkmcnt(0)); one barrier; start reading stage i+1
-// into the other fragment set; refill stage i with chunk i+4; then the 32
-// MFMAs of step i run on fragments already in registers.
+// into the other fragment set; refill stage i with chunk i+4; then the MFMAs
+// of step i run on fragments already in registers.
+//
+// What bounds a tile: the L2-to-LDS bytes and the LDS reads per MFMA fall with
+// the tile's sides (a k step of 32 takes 0.16 us on 128 x 128 tiles, of them
+// 0.11 us MFMA at 2.4 GHz, and 0.62 us on 256 x 256, 0.43 us MFMA), against
+// how evenly the tiles fill the CUs and how long a tile's fill and epilogue
+// stand alone (4.9 against 11.7 us; the smaller tiles share a CU in twos).
+// Hence the four tiles and the cost model that picks one (big_tile). Measured,
+// us, 256-row tiles alone before: 3056 x 6144 x 1536 91 -> 62 (128 x 192),
+// 3056 x 1536 x 6144 128 -> 61 (was 64 x 64), 4096 x 768 x 3072 57 -> 24
+// (128 x 128), 8192 x 1536 x 6144 165 -> 128 (1.2 PFLOP/s).
 //
 // The MFMA takes the weight block as its first operand, so a lane's result
 // is row m0 + l % 32 and, per group of four registers, four consecutive
 // columns: fp32 outputs are written as float4, and the bf16 fragment-order
 // output (ReLU^2, the next GEMM's operand) goes through a 32 x 32 LDS
-// transpose per wave (8-byte writes, 16-byte reads).
+// transpose per wave (8-byte writes, 16-byte reads). The QKV projection takes
+// 128 x 128 tiles, one head each (1904-8192 rows x 4608 x 1536, with its
+// attention prologue: 49-126 us, 59-167 us on 256 x 256).
 //
-// Tile order: tiles are grouped by 4 M tiles (N tile slower within a group)
-// and dealt to the eight XCDs in contiguous ranges, so the ~32 workgroups
-// an XCD runs at once cover about 4 M tiles x 8 N tiles and share their
-// operand slabs in that XCD's L2.
+// Tile order: tiles are grouped by 1024 rows of M tiles (N tile slower within
+// a group) and dealt to the eight XCDs in contiguous ranges, so that the
+// workgroups an XCD runs at once share their operand slabs in its L2.
 #ifndef FC_BIG_M
 #define FC_BIG_M 1024
 #endif
@@ -1269,9 +1275,9 @@ __global__ __launch_bounds__(256) void k_gemm_ring(const bf16_t* __restrict__ A,
 #ifndef FC_BIG_HEAD_M
 #define FC_BIG_HEAD_M 200
 #endif
-template <int NB>
+template <int MB, int NB>
 struct BigStage {
-  uint4 a[16][64];
+  uint4 a[4 * MB][64];
   uint4 w[4 * NB][64];
 };
 template <int EPI>
@@ -1323,75 +1329,66 @@ __device__ __forceinline__ void big_store4(const Epi& e, int m, int n, float v0,
     epi_apply<EPI, true>(e, m, n + 3, v3);
   }
 }
-template <int EPI, int NB>
-__global__ __launch_bounds__(256) void k_gemm_big(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
-                                                  int Mcap, const int* __restrict__ Mdev, int N, int K, int ntiles,
-                                                  int mtiles, int per_xcd, int S, Epi e) {
-  // NB 32-column blocks per wave: tile 256 x 64 NB (NB = 4: 256 x 256; NB = 3: 256 x 192)
-  constexpr int NSTG = 4, GM = 4, NT = 64 * NB;
-  static_assert(NB == 3 || NB == 4, "tile widths 192 and 256");
-  static_assert(EPI != EPI_QKV || NB == 4, "the QKV epilogue needs one head (128 columns) per wave");
-  __shared__ BigStage<NB> s0, s1, s2, s3;
-  // tile of this workgroup. Unsplit: XCD id % 8 takes grouped tiles
-  // [x per_xcd, (x + 1) per_xcd). Split 8 ways in K (EPI_PARTIAL): XCD x
-  // takes split x, whose workgroups share its A and W slabs in that XCD's L2,
-  // M tile slowest, so the live tiles (below the device row count) come
-  // first and the plan keeps them within the XCD's 32 CUs.
-  int sp, nt, mt;
-  if (S == 8) {
-    sp = blockIdx.x & 7;
-    const int j = blockIdx.x >> 3;
-    if (j >= ntiles * mtiles) return;
-    mt = j / ntiles;
-    nt = j - mt * ntiles;
-  } else {
-    const int t = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per_xcd || t >= ntiles * mtiles) return;
-    const int grp = t / (GM * ntiles), rr = t - grp * GM * ntiles;
-    const int gm = min(GM, mtiles - grp * GM);
-    nt = rr / gm;
-    mt = grp * GM + rr % gm;
-    sp = 0;
-  }
+// NTW: the weights stream non-temporally (one M tile: each byte is read once).
+template <int EPI, int MB, int NB, bool NTW = false>
+__global__ __launch_bounds__(256, MB == 2 ? 2 : 1) void k_gemm_big(
+    const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int Mcap, const int* __restrict__ Mdev, int N, int K,
+    int ntiles, int S, Epi e) {
+  // MB 32-row by NB 32-column blocks per wave, 2 x 2 waves: tile 64 MB x 64 NB
+  constexpr int NSTG = 4, GM = 16 / MB, MT = 64 * MB, NT = 64 * NB;
+  static_assert((MB == 2 || MB == 4) && NB >= 2 && NB <= 4, "tile shapes");
+  static_assert(EPI != EPI_QKV || NB == 2, "the QKV epilogue takes one head (128 columns) per tile");
+  typedef BigStage<MB, NB> Stage;
+  __shared__ Stage s0, s1, s2, s3;
+  // tile of this workgroup: XCD id % 8 takes an eighth of the live tiles (below
+  // the device row count) of all splits, split-major, so that the workgroups
+  // of a split share their A and W slabs in few XCDs' L2 (S = 8: split x on
+  // XCD x). Within a split, groups of GM M tiles, N tile slower in a group.
   const int M = Mdev ? min(*Mdev, Mcap) : Mcap;
-  const int m0 = mt * 256;
-  if (m0 >= M) return;
+  const int mtiles = (M + MT - 1) / MT, tiles = ntiles * mtiles;
+  const int per_xcd = (tiles * S + 7) / 8;
+  const int t = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per_xcd || t >= tiles * S) return;
+  const int sp = t / tiles, tt = t - sp * tiles;
+  const int grp = tt / (GM * ntiles), rr = tt - grp * GM * ntiles;
+  const int gm = min(GM, mtiles - grp * GM);
+  const int nt = rr / gm, mt = grp * GM + rr % gm;
+  const int m0 = mt * MT;
   const int n0 = nt * NT;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   const int64_t KS32 = K >> 5;
-  // this split's 32-deep k steps [c0, c0 + C); the host makes C a multiple of 4
+  // this split's 32-deep k steps [c0, c0 + C)
   const int c0 = (int)(sp * KS32 / S), C = (int)((sp + 1) * KS32 / S) - c0;
   const int last_blk = (M - 1) >> 4;
-  // this wave's loads: activation row blocks 4 wave .. +3 and weight column blocks NB wave .. +NB-1
-  const bf16_t* ab[4];
+  // this wave's loads: activation row blocks MB wave .. +MB-1 and weight column blocks NB wave .. +NB-1
+  const bf16_t* ab[MB];
   const bf16_t* wb[NB];
 #pragma unroll
-  for (int u = 0; u < 4; ++u)
-    ab[u] = A + ((int64_t)min(m0 / 16 + 4 * wave + u, last_blk) * KS32 + c0) * 512 + lane * 8;
+  for (int u = 0; u < MB; ++u)
+    ab[u] = A + ((int64_t)min(m0 / 16 + MB * wave + u, last_blk) * KS32 + c0) * 512;
 #pragma unroll
-  for (int u = 0; u < NB; ++u) wb[u] = W + ((int64_t)(n0 / 16 + NB * wave + u) * KS32 + c0) * 512 + lane * 8;
+  for (int u = 0; u < NB; ++u) wb[u] = W + ((int64_t)(n0 / 16 + NB * wave + u) * KS32 + c0) * 512;
   // this lane's 32x32x16 operand slot: 16-row block offset and lane slot (half 0; +32 for half 1)
   const int sub = (lane & 31) >> 4, slot = (lane & 15) + 16 * (lane >> 5);
-  f32x16 acc[4][NB];
+  f32x16 acc[MB][NB];
 #pragma unroll
-  for (int p = 0; p < 4; ++p)
+  for (int p = 0; p < MB; ++p)
 #pragma unroll
     for (int q = 0; q < NB; ++q)
 #pragma unroll
       for (int x = 0; x < 16; ++x) acc[p][q][x] = 0.f;
-  constexpr int NV = (4 + NB) * (NSTG - 2);
+  constexpr int NV = (MB + NB) * (NSTG - 2);
   static_assert(NV < 64, "vmcnt range");
+  const uint32_t voff = lane * 16;
 #define BIG_ISSUE(S, c_)                                                                                      \
   {                                                                                                           \
     const int c = min((c_), C - 1); /* past the end: harmless re-reads into an unread stage */                \
-    _Pragma("unroll") for (int u = 0; u < 4; ++u)                                                             \
-      __builtin_amdgcn_global_load_lds((const void*)(ab[u] + (int64_t)c * 512),                              \
-                                       (__attribute__((address_space(3))) void*)&S.a[4 * wave + u][0], 16, 0, 0); \
+    const uint32_t la_ = LDS_ADDR(S) + MB * 1024 * wave, lw_ = LDS_ADDR(S) + 4096 * MB + NB * 1024 * wave;    \
+    _Pragma("unroll") for (int u = 0; u < MB; ++u)                                                            \
+      lds_load_1k(ab[u] + (int64_t)c * 512, voff, la_ + 1024 * u);                                            \
     _Pragma("unroll") for (int u = 0; u < NB; ++u)                                                            \
-      __builtin_amdgcn_global_load_lds((const void*)(wb[u] + (int64_t)c * 512),                              \
-                                       (__attribute__((address_space(3))) void*)&S.w[NB * wave + u][0], 16, 0,   \
-                                       EPI == EPI_SOFTCAP && FC_BIG_LM_NT ? 2 : 0);                          \
+      lds_load_1k<NTW>(wb[u] + (int64_t)c * 512, voff, lw_ + 1024 * u);        \
   }
 #define BIG_SYNC(NVW)                                                                                         \
   {                                                                                                           \
@@ -1409,43 +1406,38 @@ __global__ __launch_bounds__(256) void k_gemm_big(const bf16_t* __restrict__ A, 
     _Pragma("unroll") for (int h = 0; h < 2; ++h) {                                                           \
       _Pragma("unroll") for (int b = 0; b < NB; ++b)                                                          \
         WF[h][b] = __builtin_bit_cast(v4u, S.w[2 * NB * wn + 2 * b + sub][slot + 32 * h]);                    \
-      _Pragma("unroll") for (int b = 0; b < 4; ++b)                                                           \
-        AF[h][b] = __builtin_bit_cast(v4u, S.a[8 * wm + 2 * b + sub][slot + 32 * h]);                         \
+      _Pragma("unroll") for (int b = 0; b < MB; ++b)                                                          \
+        AF[h][b] = __builtin_bit_cast(v4u, S.a[2 * MB * wm + 2 * b + sub][slot + 32 * h]);                    \
     }                                                                                                         \
   }
 #define BIG_MMA(WF, AF)                                                                                       \
   {                                                                                                           \
     _Pragma("unroll") for (int h = 0; h < 2; ++h)                                                             \
-      _Pragma("unroll") for (int p = 0; p < 4; ++p)                                                           \
+      _Pragma("unroll") for (int p = 0; p < MB; ++p)                                                          \
         _Pragma("unroll") for (int q = 0; q < NB; ++q) acc[p][q] = mfma32(WF[h][q], AF[h][p], acc[p][q]);     \
   }
-  // step i: SN = stage of chunk i + 1 (read now), SI = stage of chunk i (refilled with chunk i + 4)
+  // step i: SN = stage of chunk i + 1 (read now; past the last chunk a
+  // re-read that nothing uses), SI = stage of chunk i (refilled with chunk i + 4)
 #define BIG_STEP(SI, SN, WFC, AFC, WFN, AFN, i_)                                                              \
-  {                                                                                                           \
+  if ((i_) < C) {                                                                                             \
     BIG_SYNC(NV);                                                                                             \
     BIG_READ(SN, WFN, AFN);                                                                                   \
     BIG_ISSUE(SI, (i_) + NSTG);                                                                               \
     BIG_MMA(WFC, AFC);                                                                                        \
   }
-  v4u wf0[2][NB], af0[2][4], wf1[2][NB], af1[2][4];
+  v4u wf0[2][NB], af0[2][MB], wf1[2][NB], af1[2][MB];
   BIG_ISSUE(s0, 0);
   BIG_ISSUE(s1, 1);
   BIG_ISSUE(s2, 2);
   BIG_ISSUE(s3, 3);
-  BIG_SYNC(3 * (4 + NB));  // chunk 0 landed: at most the 3 later chunks' loads outstanding
+  BIG_SYNC(3 * (MB + NB));  // chunk 0 landed: at most the 3 later chunks' loads outstanding
   BIG_READ(s0, wf0, af0);
-  // C % 4 == 0 (K % 128 == 0): 4-step groups, the last one ends without a read
-  int i = 0;
-  for (; i + 4 < C; i += 4) {
+  for (int i = 0; i < C; i += NSTG) {
     BIG_STEP(s0, s1, wf0, af0, wf1, af1, i);
     BIG_STEP(s1, s2, wf1, af1, wf0, af0, i + 1);
     BIG_STEP(s2, s3, wf0, af0, wf1, af1, i + 2);
     BIG_STEP(s3, s0, wf1, af1, wf0, af0, i + 3);
   }
-  BIG_STEP(s0, s1, wf0, af0, wf1, af1, i);
-  BIG_STEP(s1, s2, wf1, af1, wf0, af0, i + 1);
-  BIG_STEP(s2, s3, wf0, af0, wf1, af1, i + 2);
-  BIG_MMA(wf1, af1);
 #undef BIG_STEP
 #undef BIG_MMA
 #undef BIG_READ
@@ -1457,47 +1449,30 @@ __global__ __launch_bounds__(256) void k_gemm_big(const bf16_t* __restrict__ A, 
   // column 32 q + 8 j + 4 (l / 32) + x
   const int rl = lane & 31, ch = 4 * (lane >> 5);
   if constexpr (EPI == EPI_QKV) {
-    // the quadrant is one head slot (128 columns) for 128 tokens: per 32
-    // tokens, stage the rows in this wave's own LDS stage (fp32), then eight
-    // lanes per token finish RoPE / QK-norm / VE gate / KV append
-    BigStage<NB>* mine = wave == 0 ? &s0 : wave == 1 ? &s1 : wave == 2 ? &s2 : &s3;
-    float(*T)[128 + 4] = (float(*)[128 + 4])mine;
-    const int hh = (n0 + 128 * wn) >> 7;
-    const int mq = m0 + 128 * wm + (lane >> 3);  // this lane's token in group p, step it: mq + 32 p + 8 it
-    int rb[4][4], rp[4][4], rt[4][4];             // their cache rows / positions / ids, loaded together
+    // the tile is one head slot: the two waves of a row half stage 16 tokens
+    // at a time in one LDS stage and finish them, eight lanes per token
+    float(*T)[128 + 4] = wm == 0 ? (float(*)[128 + 4])&s0 : (float(*)[128 + 4])&s1;
+    static_assert(sizeof(Stage) >= 16 * 132 * 4, "16 staging rows");
+    const int hh = n0 >> 7, tk = 8 * wn + (lane >> 3);
+    QkvPre pre[2 * MB];
 #pragma unroll
-    for (int p = 0; p < 4; ++p)
+    for (int u = 0; u < 2 * MB; ++u) qkv_pre_row(e.qkv, m0 + 32 * MB * wm + 16 * u + tk, M, hh, pre[u]);
 #pragma unroll
-      for (int it = 0; it < 4; ++it) {
-        QkvPre r;
-        qkv_pre_row(e.qkv, mq + 32 * p + 8 * it, M, hh, r);
-        rb[p][it] = r.b;
-        rp[p][it] = r.pos;
-        rt[p][it] = r.tok;
+    for (int u = 0; u < 2 * MB; ++u) {
+      const int m = m0 + 32 * MB * wm + 16 * u + tk;
+      qkv_pre_tab(e.qkv, m, M, hh, lane & 7, pre[u]);
+      if ((lane & 31) >> 4 == (u & 1)) {
+#pragma unroll
+        for (int q = 0; q < NB; ++q)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            *(float4*)&T[lane & 15][64 * wn + 32 * q + 8 * j + ch] =
+                float4{acc[u >> 1][q][4 * j], acc[u >> 1][q][4 * j + 1], acc[u >> 1][q][4 * j + 2],
+                       acc[u >> 1][q][4 * j + 3]};
       }
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      QkvPre pre[4];  // table / value-embedding loads of the group's 4 tokens, in flight while it is staged
-#pragma unroll
-      for (int it = 0; it < 4; ++it) {
-        pre[it].b = rb[p][it];
-        pre[it].pos = rp[p][it];
-        pre[it].tok = rt[p][it];
-        qkv_pre_tab(e.qkv, mq + 32 * p + 8 * it, M, hh, lane & 7, pre[it]);
-      }
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          *(float4*)&T[rl][32 * q + 8 * j + ch] =
-              float4{acc[p][q][4 * j], acc[p][q][4 * j + 1], acc[p][q][4 * j + 2], acc[p][q][4 * j + 3]};
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int it = 0; it < 4; ++it) {
-        const int tt = 8 * it + (lane >> 3);
-        qkv_finish(e.qkv, T[tt], m0 + 128 * wm + 32 * p + tt, M, hh, lane & 7, pre[it]);
-      }
-      __builtin_amdgcn_wave_barrier();
+      __syncthreads();
+      qkv_finish(e.qkv, T[tk], m, M, hh, lane & 7, pre[u]);
+      __syncthreads();
     }
   } else if constexpr (EPI == EPI_RELU2) {
     // bf16 fragment order: per 32 x 32 block, lane l writes row l % 32,
@@ -1507,7 +1482,7 @@ __global__ __launch_bounds__(256) void k_gemm_big(const bf16_t* __restrict__ A, 
     bf16_t* out = (bf16_t*)e.out;
     const int KB = e.ldo >> 5;
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
+    for (int p = 0; p < MB; ++p) {
 #pragma unroll
       for (int q = 0; q < NB; ++q) {
 #pragma unroll
@@ -1524,15 +1499,15 @@ __global__ __launch_bounds__(256) void k_gemm_big(const bf16_t* __restrict__ A, 
 #pragma unroll
         for (int hs = 0; hs < 2; ++hs) {
           const uint4 val = *(const uint4*)(scr + (16 * hs + (lane & 15)) * 80 + 16 * (lane >> 4));
-          const int rb = (m0 + 128 * wm + 32 * p + 16 * hs) >> 4;
+          const int rb = (m0 + 32 * MB * wm + 32 * p + 16 * hs) >> 4;
           if (16 * rb < M) *(uint4*)(out + ((int64_t)rb * KB + kb) * 512 + lane * 8) = val;
         }
       }
     }
   } else {
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const int m = m0 + 128 * wm + 32 * p + rl;
+    for (int p = 0; p < MB; ++p) {
+      const int m = m0 + 32 * MB * wm + 32 * p + rl;
       if (m < M) {
 #pragma unroll
         for (int q = 0; q < NB; ++q)
@@ -1620,36 +1595,40 @@ static void launch_ring(const void* A, const void* W, int Mcap, const int* Mdev,
                                            (const bf16_t*)A, (const bf16_t*)W, Mcap, Mdev, N, K, ntiles, S, e));
 }
 
-template <int EPI, int NB>
+template <int EPI, int MB, int NB, bool NTW = false>
 static void launch_big_e(const void* A, const void* W, int Mcap, const int* Mdev, int N, int K, int S, const Epi& e,
                          hipStream_t s) {
-  const int ntiles = N / (64 * NB), mtiles = (Mcap + 255) / 256;
-  const int per_xcd = S == 8 ? ntiles * mtiles : (ntiles * mtiles + 7) / 8;
-  hipLaunchKernelGGL((k_gemm_big<EPI, NB>), dim3(8 * per_xcd), dim3(256), 0, s, (const bf16_t*)A, (const bf16_t*)W,
-                     Mcap, Mdev, N, K, ntiles, mtiles, per_xcd, S, e);
+  const int ntiles = N / (64 * NB), mtiles = (Mcap + 64 * MB - 1) / (64 * MB);
+  const int per_xcd = (ntiles * mtiles * S + 7) / 8;
+  hipLaunchKernelGGL((k_gemm_big<EPI, MB, NB, NTW>), dim3(8 * per_xcd), dim3(256), 0, s, (const bf16_t*)A,
+                     (const bf16_t*)W, Mcap, Mdev, N, K, ntiles, S, e);
 }
-// 256-column tiles unless they leave CUs idle in a single partial wave of
-// workgroups and 192 divides N (n_embd-wide outputs: 1536 = 8 x 192)
-static int big_tile_blocks(int Mcap, int N) {
-  const int mtiles = (Mcap + 255) / 256;
-  if (N % 256 == 0 && (N / 256) * mtiles >= 240) return 4;
-  return N % 192 == 0 ? 3 : 4;
-}
-// nb: 32-column blocks per wave (3 or 4), 0 = by big_tile_blocks; S > 1 only with EPI_PARTIAL
-static void launch_big(const void* A, const void* W, int Mcap, const int* Mdev, int N, int K, int nb, int S,
+// 64 mb x 64 nb tiles; S > 1 only with EPI_PARTIAL
+static void launch_big(const void* A, const void* W, int Mcap, const int* Mdev, int N, int K, int mb, int nb, int S,
                        const Epi& e, hipStream_t s) {
-  const bool w192 = e.mode != EPI_QKV && (nb ? nb == 3 : big_tile_blocks(Mcap, N) == 3);
-#define BIG_NB(E) (w192 ? launch_big_e<E, 3>(A, W, Mcap, Mdev, N, K, S, e, s) : launch_big_e<E, 4>(A, W, Mcap, Mdev, N, K, S, e, s))
-  switch (e.mode) {
-    case EPI_STORE: BIG_NB(EPI_STORE); break;
-    case EPI_ADD: BIG_NB(EPI_ADD); break;
-    case EPI_RELU2: BIG_NB(EPI_RELU2); break;
-    case EPI_MLPOUT: BIG_NB(EPI_MLPOUT); break;
-    case EPI_PARTIAL: BIG_NB(EPI_PARTIAL); break;
-    case EPI_QKV: launch_big_e<EPI_QKV, 4>(A, W, Mcap, Mdev, N, K, 1, e, s); break;
-    default: BIG_NB(EPI_SOFTCAP); break;
+#define BIG_TILE(E)                                                                      \
+  {                                                                                      \
+    if (mb == 4 && nb == 4) launch_big_e<E, 4, 4>(A, W, Mcap, Mdev, N, K, S, e, s);      \
+    else if (mb == 4) launch_big_e<E, 4, 3>(A, W, Mcap, Mdev, N, K, S, e, s);            \
+    else if (nb == 3) launch_big_e<E, 2, 3>(A, W, Mcap, Mdev, N, K, S, e, s);            \
+    else launch_big_e<E, 2, 2>(A, W, Mcap, Mdev, N, K, S, e, s);                         \
   }
-#undef BIG_NB
+  switch (e.mode) {
+    case EPI_STORE: BIG_TILE(EPI_STORE); break;
+    case EPI_ADD: BIG_TILE(EPI_ADD); break;
+    case EPI_RELU2: BIG_TILE(EPI_RELU2); break;
+    case EPI_MLPOUT: BIG_TILE(EPI_MLPOUT); break;
+    case EPI_PARTIAL: BIG_TILE(EPI_PARTIAL); break;
+    case EPI_QKV: launch_big_e<EPI_QKV, 2, 2>(A, W, Mcap, Mdev, N, K, 1, e, s); break;  // one head per tile
+    default:
+      // the lm_head: with one M tile its weights are read once, past the
+      // caches; several M tiles share them there (4096 x 65536 x 768: 970 us
+      // with the hint, 530 without)
+      if (mb == 4 && nb == 4 && Mcap <= 256) launch_big_e<EPI_SOFTCAP, 4, 4, true>(A, W, Mcap, Mdev, N, K, S, e, s);
+      else BIG_TILE(EPI_SOFTCAP);
+      break;
+  }
+#undef BIG_TILE
 }
 
 template <int MB>
@@ -1665,9 +1644,9 @@ static void launch_la_qkv(const void* A, const void* W, int Mcap, const int* Mde
 // the K split are chosen for the typical row count Mtyp (the grid covers
 // Mcap rows; tiles past the device-side count exit at once).
 struct GemmPlan {
-  bool gemv, la, dma, big;  // VALU GEMV (fp32) / LDS-shared-A / LDS-ring / 256 x 256 (else the K-split kernel)
+  bool gemv, la, dma, big;  // VALU GEMV (fp32) / LDS-shared-A / LDS-ring / k_gemm_big (else the K-split kernel)
   bool ring;                // deep direct-load ring, 64 x 96 tiles (k_gemm_ring)
-  int mb, nb, S;       // k_gemm_ks: 16 mb x 16 nb tile; k_gemm_la, k_gemm_dma: 16 mb x 64 nb tile
+  int mb, nb, S;       // k_gemm_ks: 16 mb x 16 nb tile; k_gemm_la, k_gemm_dma: 16 mb x 64 nb; k_gemm_big: 64 mb x 64 nb
 };
 #ifndef FC_GEMM_DMA
 #define FC_GEMM_DMA 1
@@ -1696,17 +1675,52 @@ struct GemmPlan {
 #ifndef FC_MID_M
 #define FC_MID_M 832
 #endif
-// residual-stream GEMMs of verify chunks from FC_MID_M rows on the 256-row
-// tiles with a K split (MFMA-bound there: 1280 x 1536 x 6144 is 24 GFLOP)
-#ifndef FC_BIG_SPLIT
-#define FC_BIG_SPLIT 1
-#endif
 // column blocks of 64 per tile of the draft lm_head (up to 32 rows): with the
 // vocab pass in its epilogue, 32 x 128 tiles (2) measured 4.780-4.788 vs
 // 4.773-4.775 ms per cfg4 round (alternating builds)
 #ifndef FC_DRAFT_HEAD_NB
 #define FC_DRAFT_HEAD_NB 1
 #endif
+// The k_gemm_big tiles and what one of them costs a CU: fixed + per 32-deep k
+// step, in us, from sweeps of 160-8192 rows over N = 768-6144, K = 768-6144.
+// A launch takes about the tiles of the busiest CU times that, whether one or
+// two workgroups share the CU.
+struct BigTile {
+  int mb, nb;
+  float fixed, step;
+};
+static const BigTile kBigTiles[] = {{2, 2, 4.9f, 0.16f}, {2, 3, 5.9f, 0.243f}, {4, 3, 9.f, 0.48f}, {4, 4, 11.7f, 0.62f}};
+
+// From more 64 x 64 tiles than two per CU, k_gemm_big is the faster kernel
+// (us at N x K: 4608 x 1536 448 rows 11.9 vs 13.8, 640 rows 16.5 vs 15.0;
+// 1536 x 1536 1300 rows 12.6 vs 14.4, 1904 rows 20.9 vs 15.2; 768 x 768 1904
+// rows 7.9 vs 9.4, 3056 rows 13.4 vs 10.0; at 3056 rows of 6144 x 1536 134 vs 62).
+static bool big_rows(int M, int N) {
+  if (N >= 16384) return M >= FC_BIG_M && N % 128 == 0;
+  return N % 128 == 0 && (int64_t)((M + 63) / 64) * (N / 64) > 512;
+}
+
+// The cheapest tile and K split (S of at most s_max, each split's partials
+// written and read back once by the RMSNorm that sums them, at ~4 TB/s). A
+// split needs at least 8 k steps.
+static void big_tile(int M, int N, int K, int s_max, int& mb, int& nb, int& S) {
+  float best = 1e30f;
+  for (const BigTile& t : kBigTiles) {
+    if (N % (64 * t.nb) != 0) continue;
+    const int64_t tiles = (int64_t)((M + 64 * t.mb - 1) / (64 * t.mb)) * (N / (64 * t.nb));
+    for (int sp = 1; sp <= s_max && K / 32 >= 8 * sp; sp *= 2) {
+      const float part = sp > 1 ? (float)sp * M * N * 8.f / 4e6f : 0.f;
+      const float us = (float)((tiles * sp + 255) / 256) * (t.fixed + t.step * (float)(K / 32) / sp) + part;
+      if (us < best) {
+        best = us;
+        mb = t.mb;
+        nb = t.nb;
+        S = sp;
+      }
+    }
+  }
+}
+
 // Tile shape and K split by typical row count, from sweeps on MI355X at the
 // engine's shapes (N = 1536 / 4608 / 6144 / 65536, K = 1536 / 6144).
 static GemmPlan plan_gemm(int Mtyp, int N, int K, int dtype, bool can_split) {
@@ -1716,32 +1730,18 @@ static GemmPlan plan_gemm(int Mtyp, int N, int K, int dtype, bool can_split) {
     p.gemv = true;
     return p;
   }
-  if (Mtyp >= (N >= 16384 ? FC_BIG_HEAD_M : FC_BIG_M) && N % 256 == 0 && K % 128 == 0) {
-    // prefill chunks: 256 x 256 (or 256 x 192) tiles, MFMA-bound, when there
-    // are enough of them to occupy the CUs (verify-size M of ~1200 rows gives
-    // 5 M tiles: the 64-row kernels are faster there)
+  if (N >= 16384 && Mtyp >= FC_BIG_HEAD_M && N % 256 == 0 && Mtyp < FC_BIG_M) {  // the verify head
     const int mt = (Mtyp + 255) / 256;
-    const int tiles = std::max(mt * (N / 256), N % 192 == 0 ? mt * (N / 192) : 0);
-    if (tiles >= FC_BIG_MIN_TILES) {
+    if (mt * (N / 256) >= FC_BIG_MIN_TILES) {
       p.big = true;
+      p.mb = p.nb = 4;
       return p;
     }
   }
-  if (can_split && FC_BIG_SPLIT && Mtyp >= FC_MID_M && K % 1024 == 0) {
-    // large verify chunks (cfg5: 1152-1280 rows), residual-stream GEMMs with
-    // a deep K (the MLP c_proj): 256-row tiles with the K range split 8
-    // ways, one split per XCD, when a split's 24-32 output tiles fill that
-    // XCD's 32 CUs once; the next RMSNorm sums the partials
-    const int mt = (Mtyp + 255) / 256;
-    for (int nb = 4; nb >= 3; --nb) {
-      const int tiles = N % (64 * nb) == 0 ? mt * (N / (64 * nb)) : 0;
-      if (tiles >= 24 && tiles <= 32) {
-        p.big = true;
-        p.nb = nb;
-        p.S = 8;
-        return p;
-      }
-    }
+  if (big_rows(Mtyp, N)) {
+    p.big = true;
+    big_tile(Mtyp, N, K, can_split ? FC_MAX_SPLIT : 1, p.mb, p.nb, p.S);
+    return p;
   }
   const int C = K / 64;
   const int s_max = std::max(1, std::min(C / 4, FC_MAX_SPLIT));  // >= 1 chunk per wave
@@ -1844,7 +1844,7 @@ bool fc_gemm_fuses_qkv(int Mtyp, int N, int K, int dtype, int head_dim) {
   if (dtype != FC_BF16 || head_dim != 128 || N % 128 != 0 || K % 64 != 0) return false;
   if (Mtyp <= FC_QKV_TINY_M) return true;
   const GemmPlan p = plan_gemm(Mtyp, N, K, dtype, false);
-  // the QKV tile itself is k_gemm_la's 32 x 128 (64 x 128 from FC_MID_M rows), or a 128 x 128 quadrant of k_gemm_big
+  // the QKV tile itself is k_gemm_la's 32 x 128 (64 x 128 from FC_MID_M rows), or k_gemm_big's 128 x 128
   return p.big || p.dma || (p.la && p.mb == 2 && p.nb == 2);
 }
 
@@ -1889,7 +1889,8 @@ int fc_launch_gemm(const void* A, const void* W, int Mcap, const int* Mdev, int 
                "bf16 GEMM needs K % 64 == 0 and N % 32 == 0 (fragment-order operands)");
   if (e.mode == EPI_QKV) {
     FC_CHECK_ARG(fc_gemm_fuses_qkv(Mtyp, N, K, dtype, 128), "EPI_QKV needs the 32 x 128 bf16 tile");
-    if (plan_gemm(Mtyp, N, K, dtype, false).big) launch_big(A, W, Mcap, Mdev, N, K, 0, 1, e, s);
+    const GemmPlan q = plan_gemm(Mtyp, N, K, dtype, false);
+    if (q.big) launch_big(A, W, Mcap, Mdev, N, K, q.mb, q.nb, 1, e, s);
     else if (Mtyp >= FC_MID_M) launch_la_qkv<4>(A, W, Mcap, Mdev, N, K, e, s);  // 64 x 128 tiles
     else launch_la_qkv<2>(A, W, Mcap, Mdev, N, K, e, s);
     FC_LAUNCH_CHECK();
@@ -1917,9 +1918,7 @@ int fc_launch_gemm(const void* A, const void* W, int Mcap, const int* Mdev, int 
     launch_gemv<float>(A, W, Mcap, Mdev, N, K, ee, s);
   } else if (p.big) {
     FC_CHECK_ARG(ee.rms_in == nullptr && ee.xa == nullptr, "the 256 x 256 GEMM has no folded-norm epilogue");
-    FC_CHECK_ARG(p.S == 1 || (p.S == 8 && ee.mode == EPI_PARTIAL && K % 1024 == 0),
-                 "the 256 x 256 GEMM splits K only 8 ways, in multiples of 4 k steps per split");
-    launch_big(A, W, Mcap, Mdev, N, K, p.nb, p.S, ee, s);
+    launch_big(A, W, Mcap, Mdev, N, K, p.mb, p.nb, p.S, ee, s);
   } else if (p.ring) {
     if (p.mb == 2) launch_ring<2, 2, 4, 2>(A, W, Mcap, Mdev, N, K, p.S, ee, s);  // 32 x 32, 4 stages
     else launch_ring<4, 6, 5, 2>(A, W, Mcap, Mdev, N, K, p.S, ee, s);           // 64 x 96, 5 stages

@@ -1,0 +1,94 @@
+"""k_gemm_big's four tiles (128 x 128, 128 x 192, 256 x 192, 256 x 256) at
+ragged row counts and k-step counts that are not a multiple of its ring, each
+epilogue fc_gemm offers, and the QKV projection on its 128 x 128 tile."""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+from flaxchat_amd._lib import check, lib  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+def _stream():
+    return torch.cuda.current_stream().cuda_stream
+
+
+def _pack(t):
+    R, K = t.shape
+    out = torch.empty((R + 15) // 16 * 16, K, dtype=t.dtype, device="cuda")
+    check(lib().fc_pack_operand(t.data_ptr(), out.data_ptr(), R, K, _stream()), "pack")
+    return out
+
+
+# the smallest row counts past 512 tiles of 64 x 64 and ragged ones; K / 32 = 2,
+# 6, 10 (ring remainders 2), 24 and 192
+@pytest.mark.parametrize("M,N,K", [(2753, 768, 64), (2753, 768, 192), (3000, 768, 320), (4111, 1152, 768),
+                                   (16385, 128, 64), (3056, 1536, 768), (6000, 1536, 3072), (8191, 2048, 1536),
+                                   (1025, 16384, 128)])
+@pytest.mark.parametrize("epi", [0, 1, 2, 4])
+def test_large_tiles(M, N, K, epi):
+    print(f"M={M} N={N} K={K} epi={epi}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+    w = (torch.randn(N, K, device="cuda", generator=g) * 0.05).to(torch.bfloat16)
+    a, b = _pack(x), _pack(w)
+    ref = x.double() @ w.double().t()
+    # fp32 accumulation of K products: 2^-24 per add on a sum of size |x||w| sqrt(K)
+    tol = 2.0 ** -24 * K * 0.05 * 3
+    if epi == 2:
+        out = torch.zeros((M + 15) // 16 * 16, N, device="cuda", dtype=torch.bfloat16)
+    elif epi == 1:
+        base = torch.randn(M, N, device="cuda", generator=g)
+        out = base.clone()
+    else:
+        out = torch.full((M + 1, N), 7.0, device="cuda")
+    check(lib().fc_gemm(a.data_ptr(), b.data_ptr(), out.data_ptr(), M, N, K, 1, epi, _stream()), "fc_gemm")
+    if epi == 0:
+        assert float((out[:M] - ref).abs().max()) <= tol and bool((out[M] == 7.0).all())
+    elif epi == 1:
+        assert float((out - (ref + base)).abs().max()) <= tol + 2.0 ** -21
+    elif epi == 4:
+        # the bf16 kernels' softcap is within 5e-6 of 15 tanh(z / 15)
+        assert float((out[:M] - 15 * torch.tanh(ref / 15)).abs().max()) <= tol + 1e-5 and bool((out[M] == 7.0).all())
+    else:
+        from flaxchat_amd.torch_ops import frag_to_rows
+        got, want = frag_to_rows(out, M).double(), torch.relu(ref) ** 2
+        assert bool(((got - want).abs() <= want * 2.0 ** -8 + 2 * tol * ref.abs() + 1e-6).all())
+
+
+@pytest.mark.parametrize("M,D,kv", [(1000, 1536, 12), (1301, 1536, 4), (2050, 768, 6)])
+def test_qkv_tile_matches_the_separate_prologue(M, D, kv):
+    """fc_attn_qkv's fused tile against the plain GEMM and fc_attn_prologue:
+    the same q and cache to one bf16 ulp (different order of the sums)."""
+    import flaxchat_amd.torch_ops  # noqa: F401
+    from flaxchat_amd.config import GPTConfig
+    from flaxchat_amd.runtime import DeviceCache, DeviceModel
+    ops = torch.ops.flaxchat_mi355x
+    print(f"M={M} D={D} kv={kv}", flush=True)
+    cfg = GPTConfig(sequence_len=512, vocab_size=1000, n_layer=2, n_head=D // 128, n_kv_head=kv, n_embd=D)
+    dm = DeviceModel.random_init(cfg, seed=1, dtype="bf16")
+    B, per = 4, (M + 3) // 4
+    g = torch.Generator(device="cuda").manual_seed(M)
+    tok = torch.randint(0, 1000, (M,), device="cuda", dtype=torch.int32, generator=g)
+    i = torch.arange(M, device="cuda")
+    row, pos = (i // per).int(), (i % per).int()
+    row[5] = -1                                   # skipped token
+    h = torch.randn((M + 15) // 16 * 16, D, device="cuda", generator=g).to(torch.bfloat16)
+    addr = ctypes.addressof(dm.desc)
+    got, want = DeviceCache(dm, B, per + 32), DeviceCache(dm, B, per + 32)
+    for layer in (0, 1):                          # without and with a value embedding
+        assert lib().fc_attn_qkv_workspace_bytes(ctypes.byref(dm.desc), M, 0) == 0
+        q = ops.attn_qkv(addr, layer, got.k, got.v, h, tok, row, pos)
+        qkv = torch.empty(M, (dm.H + 2 * dm.G) * 128, device="cuda")
+        check(lib().fc_gemm(h.data_ptr(), dm.t["layers"][layer]["wqkv"].data_ptr(), qkv.data_ptr(), M, qkv.shape[1],
+                            D, 1, 0, _stream()), "fc_gemm")
+        q2 = ops.attn_prologue(addr, layer, want.k, want.v, qkv, h, tok, row, pos)
+        keep = np.arange(M) != 5
+        np.testing.assert_allclose(q.float().cpu().numpy()[keep], q2.float().cpu().numpy()[keep], rtol=2.0 ** -7,
+                                   atol=2.0 ** -9)
+    for a, b in ((got.k, want.k), (got.v, want.v)):
+        np.testing.assert_allclose(a.float().cpu().numpy(), b.float().cpu().numpy(), rtol=2.0 ** -7, atol=2.0 ** -9)
