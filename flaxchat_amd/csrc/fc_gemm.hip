@@ -36,21 +36,19 @@
 #include "fc_common.h"
 #include "fc_internal.h"
 
-// 15 tanh(v / 15) in the bf16 kernels' epilogues. tanh(x) = sign(x) (1 - 2 /
-// (e^{2|x|} + 1)) with e^{2|x|} from the hardware base-2 exponential and the
-// reciprocal from v_rcp_f32 (about 1 ulp each); below |x| = 1/16, where that
-// form cancels, the series x - x^3/3 + 2x^5/15 (truncation < 3e-10). The
-// capped value is within ~5e-6 of 15 tanhf(v / 15), far below the bf16
-// GEMM's own rounding, at about a third of the instructions of the
-// IEEE divide and tanhf. The fp32 kernels keep the exact form.
+// 15 tanh(v / 15) in the bf16 kernels' epilogues: 15 - 30 / (e^{2v/15} + 1),
+// with the hardware base-2 exponential and reciprocal (about 1 ulp each; at
+// their limits the form gives +-15 by itself); below |v| = 15/16, where it
+// cancels, the series v (1 - x^2/3 + 2x^4/15) of x = v / 15 (truncation <
+// 3e-9). The capped value is within ~5e-6 of 15 tanhf(v / 15), far below the
+// bf16 GEMM's own rounding, in 11 instructions. The fp32 kernels keep the
+// exact form.
 __device__ __forceinline__ float softcap15_fast(float v) {
-  const float x = v * (1.f / 15.f);
-  const float a = fabsf(x);
-  const float x2 = x * x;
-  const float ts = x * fmaf(x2, fmaf(x2, 2.f / 15.f, -1.f / 3.f), 1.f);
-  const float ex = __builtin_amdgcn_exp2f(a * 2.8853900817779268f);  // e^{2a}
-  const float tl = copysignf(1.f - 2.f * __builtin_amdgcn_rcpf(ex + 1.f), x);
-  return 15.f * (a < 0.0625f ? ts : tl);
+  const float v2 = v * v;
+  const float ts = v * fmaf(v2, fmaf(v2, 2.f / (15.f * 50625.f), -1.f / (3.f * 225.f)), 1.f);
+  const float ex = __builtin_amdgcn_exp2f(v * (2.8853900817779268f / 15.f));  // e^{2v/15}
+  const float tl = fmaf(-30.f, __builtin_amdgcn_rcpf(ex + 1.f), 15.f);
+  return fabsf(v) < 0.9375f ? ts : tl;
 }
 
 // FAST: the bf16 kernels' softcap (softcap15_fast); the fp32 kernel uses tanhf.
@@ -1280,53 +1278,54 @@ struct BigStage {
   uint4 a[4 * MB][64];
   uint4 w[4 * NB][64];
 };
+// Epilogue inputs of a 32 x 32 output block: the lane's four float4 of x and
+// of the second operand (EPI_MLPOUT: x0, or the backout capture at the end).
+struct BigIn {
+  float4 x[4], z[4];
+};
 template <int EPI>
-__device__ __forceinline__ void big_store4(const Epi& e, int m, int n, float v0, float v1, float v2, float v3,
-                                           int split) {
+__device__ __forceinline__ void big_load(const Epi& e, int m, int n, int M, BigIn& in) {
+  if constexpr (EPI == EPI_ADD || EPI == EPI_MLPOUT) {
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+      const int64_t i = (int64_t)min(m + 8 * it, M - 1) * e.ldo + n;
+      in.x[it] = *(const float4*)((const float*)e.out + i);
+      if constexpr (EPI == EPI_MLPOUT)
+        if (!e.last || !e.capture) in.z[it] = *(const float4*)((e.last ? e.xb : e.x0) + i);
+    }
+  }
+}
+template <int EPI>
+__device__ __forceinline__ void big_store4(const Epi& e, int m, int n, float4 v, float4 x, float4 z, int split,
+                                           float* logit_row) {
   if constexpr (EPI == EPI_STORE) {
-    *(float4*)((float*)e.out + (int64_t)m * e.ldo + n) = float4{v0, v1, v2, v3};
+    *(float4*)((float*)e.out + (int64_t)m * e.ldo + n) = v;
   } else if constexpr (EPI == EPI_ADD) {
-    float4* o = (float4*)((float*)e.out + (int64_t)m * e.ldo + n);
-    const float4 x = *o;
-    *o = float4{x.x + v0, x.y + v1, x.z + v2, x.w + v3};
+    *(float4*)((float*)e.out + (int64_t)m * e.ldo + n) = float4{x.x + v.x, x.y + v.y, x.z + v.z, x.w + v.w};
   } else if constexpr (EPI == EPI_MLPOUT) {
     const int64_t i = (int64_t)m * e.ldo + n;
     float4* xp = (float4*)((float*)e.out + i);
-    const float4 x = *xp;
-    const float4 t = float4{x.x + v0, x.y + v1, x.z + v2, x.w + v3};  // engine.py:161
-    float4 xb = float4{0.f, 0.f, 0.f, 0.f};
-    if (e.capture) {                                                   // engine.py:164
-      *(float4*)(e.xb + i) = t;
-      xb = t;
-    } else if (e.last) {
-      xb = *(const float4*)(e.xb + i);
-    }
-    if (e.last) {                                                      // engine.py:166
+    const float4 t = float4{x.x + v.x, x.y + v.y, x.z + v.z, x.w + v.w};  // engine.py:161
+    if (e.capture) *(float4*)(e.xb + i) = t;                               // engine.py:164
+    if (e.last) {                                                          // engine.py:166
+      const float4 xb = e.capture ? t : z;
       *xp = float4{t.x - e.lb * xb.x, t.y - e.lb * xb.y, t.z - e.lb * xb.z, t.w - e.lb * xb.w};
-    } else {                                                           // engine.py:94
-      const float4 x0 = *(const float4*)(e.x0 + i);
-      *xp = float4{e.r * t.x + e.a * x0.x, e.r * t.y + e.a * x0.y, e.r * t.z + e.a * x0.z, e.r * t.w + e.a * x0.w};
+    } else {                                                               // engine.py:94
+      *xp = float4{e.r * t.x + e.a * z.x, e.r * t.y + e.a * z.y, e.r * t.z + e.a * z.z, e.r * t.w + e.a * z.w};
     }
   } else if constexpr (EPI == EPI_PARTIAL) {  // split-K partial, finished by the next RMSNorm
-    *(float4*)(e.part + ((int64_t)split * e.part_rows + m) * e.ldo + n) = float4{v0, v1, v2, v3};
+    *(float4*)(e.part + ((int64_t)split * e.part_rows + m) * e.ldo + n) = v;
   } else if constexpr (EPI == EPI_SOFTCAP) {  // logits row (m / n_out, m % n_out), columns past V dropped
-    const int b = m / e.n_out, rr = m - b * e.n_out;
-    float* o = (float*)e.out + (int64_t)b * e.row_stride + (int64_t)rr * e.V + n;
-    const float t0 = softcap15_fast(v0), t1 = softcap15_fast(v1);
-    const float t2 = softcap15_fast(v2), t3 = softcap15_fast(v3);
+    float* o = logit_row + n;
+    const float4 t = float4{softcap15_fast(v.x), softcap15_fast(v.y), softcap15_fast(v.z), softcap15_fast(v.w)};
     if (n + 3 < e.V && (((uintptr_t)o) & 15) == 0) {
-      *(float4*)o = float4{t0, t1, t2, t3};
+      *(float4*)o = t;
     } else {
-      if (n < e.V) o[0] = t0;
-      if (n + 1 < e.V) o[1] = t1;
-      if (n + 2 < e.V) o[2] = t2;
-      if (n + 3 < e.V) o[3] = t3;
+      if (n < e.V) o[0] = t.x;
+      if (n + 1 < e.V) o[1] = t.y;
+      if (n + 2 < e.V) o[2] = t.z;
+      if (n + 3 < e.V) o[3] = t.w;
     }
-  } else {
-    epi_apply<EPI, true>(e, m, n, v0);
-    epi_apply<EPI, true>(e, m, n + 1, v1);
-    epi_apply<EPI, true>(e, m, n + 2, v2);
-    epi_apply<EPI, true>(e, m, n + 3, v3);
   }
 }
 // NTW: the weights stream non-temporally (one M tile: each byte is read once).
@@ -1505,16 +1504,58 @@ __global__ __launch_bounds__(256, MB == 2 ? 2 : 1) void k_gemm_big(
       }
     }
   } else {
+    // per 32 x 32 block through this wave's LDS scratch (rows of 36 floats): a
+    // lane then holds row lane / 8 + 8 it, columns 4 (lane % 8) .. +3, so each
+    // access covers whole 128-byte lines of 8 rows. From the accumulators it
+    // would be 32 bytes of 32 rows: with rows a power of two apart (logits of
+    // 65536 entries) the lines left the L2 in pieces (4096 x 65536 x 768 with
+    // the softcap: 970 us, 727 so, 640 with the softcap's shorter form; the MLP
+    // c_proj's residual update 3056 x 1536 x 6144 87 -> 65). The next block's residual inputs are loaded
+    // before this block's stores, which would otherwise stand ahead of them.
+    // Block k + 1 is read back while block k is finished, k + 2 written.
+    float* scr = (float*)(wave == 0 ? &s0 : wave == 1 ? &s1 : wave == 2 ? &s2 : &s3);
+    constexpr int NBLK = MB * NB, SCR = 32 * 36;
+    static_assert(sizeof(Stage) >= 2 * SCR * 4, "a wave's two scratch blocks");
+    const int mr = m0 + 32 * MB * wm + (lane >> 3), nc = n0 + 32 * NB * wn + 4 * (lane & 7);
+    BigIn in[2];
+    float4 v[2][4];
+    float* lrow[4] = {nullptr, nullptr, nullptr, nullptr};  // EPI_SOFTCAP: the lane's four logits rows
+    auto put = [&](int k) {
 #pragma unroll
-    for (int p = 0; p < MB; ++p) {
-      const int m = m0 + 32 * MB * wm + 32 * p + rl;
-      if (m < M) {
+      for (int j = 0; j < 4; ++j)
+        *(float4*)(scr + (k & 1) * SCR + rl * 36 + 8 * j + ch) =
+            float4{acc[k / NB][k % NB][4 * j], acc[k / NB][k % NB][4 * j + 1], acc[k / NB][k % NB][4 * j + 2],
+                   acc[k / NB][k % NB][4 * j + 3]};
+    };
+    auto get = [&](int k) {
 #pragma unroll
-        for (int q = 0; q < NB; ++q)
+      for (int it = 0; it < 4; ++it)
+        v[k & 1][it] = *(const float4*)(scr + (k & 1) * SCR + (8 * it + (lane >> 3)) * 36 + 4 * (lane & 7));
+      big_load<EPI>(e, mr + 32 * (k / NB), nc + 32 * (k % NB), M, in[k & 1]);
+    };
+    put(0);
+    __builtin_amdgcn_wave_barrier();
+    get(0);
+    put(1);
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
-            big_store4<EPI>(e, m, n0 + 32 * NB * wn + 32 * q + 8 * j + ch, acc[p][q][4 * j], acc[p][q][4 * j + 1],
-                            acc[p][q][4 * j + 2], acc[p][q][4 * j + 3], sp);
+    for (int k = 0; k < NBLK; ++k) {
+      const int p = k / NB, q = k % NB;
+      __builtin_amdgcn_wave_barrier();
+      if (k + 1 < NBLK) get(k + 1);
+      __builtin_amdgcn_wave_barrier();
+      if (k + 2 < NBLK) put(k + 2);
+      if constexpr (EPI == EPI_SOFTCAP) {
+        if (q == 0)
+#pragma unroll
+          for (int it = 0; it < 4; ++it) {
+            const int m = mr + 32 * p + 8 * it, b = m / e.n_out;
+            lrow[it] = (float*)e.out + (int64_t)b * e.row_stride + (int64_t)(m - b * e.n_out) * e.V;
+          }
+      }
+#pragma unroll
+      for (int it = 0; it < 4; ++it) {
+        const int m = mr + 32 * p + 8 * it;
+        if (m < M) big_store4<EPI>(e, m, nc + 32 * q, v[k & 1][it], in[k & 1].x[it], in[k & 1].z[it], sp, lrow[it]);
       }
     }
   }
@@ -1622,8 +1663,7 @@ static void launch_big(const void* A, const void* W, int Mcap, const int* Mdev, 
     case EPI_QKV: launch_big_e<EPI_QKV, 2, 2>(A, W, Mcap, Mdev, N, K, 1, e, s); break;  // one head per tile
     default:
       // the lm_head: with one M tile its weights are read once, past the
-      // caches; several M tiles share them there (4096 x 65536 x 768: 970 us
-      // with the hint, 530 without)
+      // caches; several M tiles share them there
       if (mb == 4 && nb == 4 && Mcap <= 256) launch_big_e<EPI_SOFTCAP, 4, 4, true>(A, W, Mcap, Mdev, N, K, S, e, s);
       else BIG_TILE(EPI_SOFTCAP);
       break;
