@@ -175,9 +175,6 @@ __device__ __forceinline__ f32x4 mfma16a(uint4 a, uint4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
                                                   0, 0);
 }
-__device__ __forceinline__ uint32_t pack2bf(float lo, float hi) {
-  return (uint32_t)f2bf(lo) | ((uint32_t)f2bf(hi) << 16);
-}
 
 // One 32-key tile of one wave: scores S^T = K Q^T, online softmax update,
 // O^T += V^T P^T (see the kernel comment).
@@ -535,52 +532,68 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn_mfma_qb(const bf16_t* __res
 }
 
 // Prefill attention on the 32x32x16 MFMA. A workgroup owns 128 query
-// columns of one (row, KV group), 32 per wave. The 32-key K / V tiles of the
-// group's key range go through a 3-stage LDS ring by direct loads (each wave
-// 4 of a tile's 16 blocks of 1 KB), so a tile is read once per 128 columns.
-// Per tile a wave computes S^T = K Q^T (32 keys x its 32 columns; lane l
-// holds column l % 32 and 16 of the keys), the online softmax in registers
-// (one swap with lane l ^ 32 per max), then O^T += V^T P^T (4 x 32 dims); the
-// P operand of a 16-key half takes 4 keys from the lane and 4 from lane
-// l ^ 32. Both K and V are read from LDS in their cache layouts with
-// lane-dependent addresses. Waves skip the tiles outside their own key range
-// but take part in every load and barrier.
+// columns of one (row, KV group), 32 per wave, and walks the group's key range
+// in steps of 64 keys through two LDS stages: the next step's K and V load
+// while this one computes, so a key is read once per 128 columns and a step
+// has one barrier. Per step a wave computes S^T = K Q^T (two 32-key tiles x
+// its 32 columns), one online softmax update in registers, then O^T += V^T P^T
+// (4 x 32 dims).
+//
+// Operand order: the direct loads put every matrix-core operand into LDS in
+// lane order (64 lanes x 16 bytes), each lane fetching its own 16 bytes, so
+// that every LDS read is 1 KB in a row, free of bank conflicts (in the caches'
+// own order the V reads met four to a bank). The rows of the K operand are
+// taken in the order that leaves lane l with keys 16 kh + 8 (l / 32) .. +7 of
+// its column in registers 8 kh .. +7: the P operand of a 16-key half as it
+// stands, with no exchange between lanes.
+//
+// What bounds it: per 32 keys x 32 columns 512 MFMA cycles against ~540 VALU
+// (256 of them the exponentials), overlapped by the two waves of a SIMD; hence
+// the output is rescaled only in steps that raise some column's maximum.
+// 8 rows x 500-1000 queries, 12 heads, window 1024: 112 -> 70 us (before: 32 keys
+// per barrier, operands in the caches' order, an exchange per P operand).
+//
+// Workgroups: all column blocks of a (row, group) on one XCD (its K and V in
+// one L2), the last blocks, which see the most keys, first.
 struct PfStage {
-  uint4 k[8][64];  // one 32-key block of the K cache (8 KB)
-  uint4 v[512];    // one 32-key block of the V cache: [128 dims][32 keys] (8 KB)
+  uint4 k[2][8][64];  // [32-key tile][16-dim slice][lane]
+  uint4 v[2][8][64];  // [32-key tile][2 (dim / 32) + key half][lane]
 };
 __global__ __launch_bounds__(256, 2) void k_attn_pf(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
                                                  const bf16_t* __restrict__ vc, bf16_t* __restrict__ y, int H, int G,
                                                  int cap, const int* __restrict__ row_off,
                                                  const int* __restrict__ start, int max_per_row, int Mcap,
-                                                 int window, float scale_log2) {
+                                                 int window, float scale_log2, int nbg, int nblk) {
   constexpr int HD = 128;
-  __shared__ PfStage st0, st1, st2;
-  const int bg = blockIdx.y, b = bg / G, g = bg - b * G, rep = H / G;
+  __shared__ PfStage st0, st1;
+  const int nbgl = (nbg + 7) >> 3, jj = blockIdx.x >> 3;
+  const int bg = (jj % nbgl) * 8 + (blockIdx.x & 7);
+  if (bg >= nbg) return;
+  const int b = bg / G, g = bg - b * G, rep = H / G;
   const RowSpan sp = row_span(row_off, b, max_per_row, Mcap);
   const int base = sp.base, n = sp.n, s0 = start[b];
   const int ncol = n * rep;
-  const int c0 = blockIdx.x * 128;
+  const int c0 = (nblk - 1 - jj / nbgl) * 128;
   if (c0 >= ncol) return;  // the whole workgroup
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int hl = lane >> 5;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hl = lane >> 5, kk = lane & 31;
   // the workgroup's key range
   const int lcol = min(c0 + 127, ncol - 1);
   const int kbeg = window > 0 ? max(0, s0 + c0 / rep - window) : 0;
   const int kend = min(s0 + lcol / rep + 1, cap);
   const int t0 = kbeg & ~31;
-  const int ntiles = (kend - t0 + 31) >> 5;
+  const int ntiles = (kend - t0 + 31) >> 5, nstep = (ntiles + 1) >> 1;
   // this wave's columns and key range
   const int wc0 = c0 + 32 * wave;
   const bool wact = wc0 < ncol;
   const int w_hi = wact ? s0 + min(wc0 + 31, ncol - 1) / rep : -1;
   const int w_lo = window > 0 ? max(0, s0 + wc0 / rep - window) : 0;
-  // tiles inside [w_full_lo, w_full_hi] are visible to every column of the wave (no masks)
+  // keys inside [w_full_lo, w_full_hi] are visible to every column of the wave (no masks)
   const bool wfull = wc0 + 31 < ncol;
   const int w_full_hi = s0 + wc0 / rep;  // the first column's position
   const int w_full_lo = window > 0 ? max(0, s0 + (wc0 + 31) / rep - window) : 0;
   // this lane's column (query)
-  const int col = wc0 + (lane & 31);
+  const int col = wc0 + kk;
   const bool cvalid = col < ncol;
   const int j = cvalid ? col / rep : 0;
   const int head = g * rep + (cvalid ? col - (col / rep) * rep : 0);
@@ -592,9 +605,12 @@ __global__ __launch_bounds__(256, 2) void k_attn_pf(const bf16_t* __restrict__ q
 #pragma unroll
     for (int h = 0; h < 8; ++h) qf[h] = cvalid ? *(const v4u*)(qr + 16 * h) : v4u{0u, 0u, 0u, 0u};
   }
-  // LDS slots this lane reads: K (block, slot) per 16-dim slice h; V uint4 index per (dims block, key half)
-  const int kk = lane & 31;
-  const int kcc = (kk >> 2) & 1, kr = ((kk >> 3) << 2) | (kk & 3);
+  // byte offsets of this lane's 16 bytes: K operand row kk is key
+  // 16 (kk / 16) + 8 ((kk / 4) % 2) + 4 ((kk / 8) % 2) + kk % 4 of the tile (its
+  // place in a K block: see kblk_idx), V operand row kk is dim kk of 32
+  const int key = ((kk >> 4) << 4) | (((kk >> 2) & 1) << 3) | (((kk >> 3) & 1) << 2) | (kk & 3);
+  const uint32_t koff = 16u * (uint32_t)((((key >> 2) & 1) << 6) + ((key >> 3) << 2) + (key & 3) + 16 * hl);
+  const uint32_t voff = 16u * (uint32_t)(4 * kk + hl);
   const bf16_t* kbase = kc + (int64_t)bg * cap * HD;
   const bf16_t* vbase = vc + (int64_t)bg * (cap / 32) * HD * 32;
   f32x16 O[4];
@@ -603,105 +619,94 @@ __global__ __launch_bounds__(256, 2) void k_attn_pf(const bf16_t* __restrict__ q
 #pragma unroll
     for (int x = 0; x < 16; ++x) O[dd][x] = 0.f;
   float m_run = -INFINITY, l_run = 0.f;
-#define PF_ISSUE(S, t_)                                                                                    \
+  // the wave's eight loads of a step: 16-dim slices 2 wave, 2 wave + 1 of K and
+  // dims 32 wave .. +31 of V, of both tiles
+#define PF_ISSUE(S, i_)                                                                                    \
   {                                                                                                        \
-    const int kb_ = t0 + 32 * min((t_), ntiles - 1); /* past the end: harmless re-reads */                 \
-    const bf16_t* kt = kbase + (int64_t)(kb_ >> 5) * 32 * HD + lane * 8;                                   \
-    const bf16_t* vt = vbase + (int64_t)(kb_ >> 5) * HD * 32 + lane * 8;                                   \
     _Pragma("unroll") for (int u = 0; u < 2; ++u) {                                                        \
-      __builtin_amdgcn_global_load_lds((const void*)(kt + (2 * wave + u) * 512),                          \
-                                       (__attribute__((address_space(3))) void*)&S.k[2 * wave + u][0], 16, 0, 0); \
-      __builtin_amdgcn_global_load_lds((const void*)(vt + (2 * wave + u) * 512),                          \
-                                       (__attribute__((address_space(3))) void*)&S.v[64 * (2 * wave + u)], 16, 0, 0); \
+      const int64_t blk = (int64_t)((t0 >> 5) + min(2 * (i_) + u, ntiles - 1)) * 32 * HD; /* past the end: harmless re-reads */ \
+      const bf16_t* kt = kbase + blk + 1024 * wave;                                                        \
+      const bf16_t* vt = vbase + blk + 1024 * wave;                                                        \
+      const uint32_t lk = LDS_ADDR(S.k[u][0]) + 2048 * wave, lv = LDS_ADDR(S.v[u][0]) + 2048 * wave;       \
+      lds_load_1k(kt, koff, lk);                                                                           \
+      lds_load_1k(kt + 256, koff, lk + 1024);                                                              \
+      lds_load_1k(vt, voff, lv);                                                                           \
+      lds_load_1k(vt + 16, voff, lv + 1024);                                                               \
     }                                                                                                      \
   }
 #define PF_SYNC()                                                                                          \
   {                                                                                                        \
     __builtin_amdgcn_sched_barrier(0);                                                                     \
-    __builtin_amdgcn_s_waitcnt((4 & 15) | (7 << 4) | (0 << 8)); /* vmcnt(4): the next tile may be in flight */ \
+    __builtin_amdgcn_s_waitcnt(0); /* this step's loads, issued a step ago, and this wave's LDS reads */   \
     __atomic_signal_fence(__ATOMIC_SEQ_CST);                                                               \
     __builtin_amdgcn_sched_barrier(0);                                                                     \
     __builtin_amdgcn_s_barrier();                                                                          \
     __builtin_amdgcn_sched_barrier(0);                                                                     \
     __atomic_signal_fence(__ATOMIC_SEQ_CST);                                                               \
   }
-#define PF_TILE(S, t_)                                                                                     \
-  {                                                                                                        \
-    const int kb = t0 + 32 * (t_);                                                                         \
-    if (wact && kb <= w_hi && kb + 31 >= w_lo) {                                                           \
-      f32x16 sa, sb;                                                                                       \
-      _Pragma("unroll") for (int x = 0; x < 16; ++x) { sa[x] = 0.f; sb[x] = 0.f; }                       \
-      _Pragma("unroll") for (int h = 0; h < 8; ++h) {                                                      \
-        const int gq = (2 * h + hl) & 3;                                                                   \
-        const v4u kf = __builtin_bit_cast(v4u, S.k[2 * (h >> 1) + kcc][kr + 16 * gq]);                    \
-        if (h & 1) sb = mfma32(kf, qf[h], sb);                                                             \
-        else sa = mfma32(kf, qf[h], sa);                                                                   \
-      }                                                                                                    \
-      float pv[16];                                                                                        \
-      float mt = -INFINITY;                                                                                \
-      if (wfull && kb >= w_full_lo && kb + 31 <= w_full_hi) {                                              \
-        _Pragma("unroll") for (int i = 0; i < 16; ++i) {                                                   \
-          pv[i] = (sa[i] + sb[i]) * scale_log2;                                                            \
-          mt = fmaxf(mt, pv[i]);                                                                           \
-        }                                                                                                  \
-      } else {                                                                                             \
-        _Pragma("unroll") for (int i = 0; i < 16; ++i) {                                                   \
-          const int key = kb + 8 * (i >> 2) + 4 * hl + (i & 3);                                            \
-          const bool ok = cvalid && key >= lo_c && key <= pos_c;                                           \
-          pv[i] = ok ? (sa[i] + sb[i]) * scale_log2 : -INFINITY;                                           \
-          mt = fmaxf(mt, pv[i]);                                                                           \
-        }                                                                                                  \
-      }                                                                                                    \
-      mt = fmaxf(mt, __shfl_xor(mt, 32, WAVE));                                                            \
-      const float m_new = fmaxf(m_run, mt);                                                                \
-      float alpha = 1.f, psum = 0.f;                                                                       \
-      if (m_new == -INFINITY) {                                                                            \
-        _Pragma("unroll") for (int i = 0; i < 16; ++i) pv[i] = 0.f;                                        \
-      } else {                                                                                             \
-        alpha = __builtin_amdgcn_exp2f(m_run - m_new);                                                     \
-        _Pragma("unroll") for (int i = 0; i < 16; ++i) {                                                   \
-          pv[i] = __builtin_amdgcn_exp2f(pv[i] - m_new);                                                   \
-          psum += pv[i];                                                                                   \
-        }                                                                                                  \
-      }                                                                                                    \
-      l_run = l_run * alpha + psum;                                                                        \
-      m_run = m_new;                                                                                       \
-      uint2 pk[4];                                                                                         \
-      _Pragma("unroll") for (int g4 = 0; g4 < 4; ++g4)                                                     \
-        pk[g4] = uint2{pack2bf(pv[4 * g4], pv[4 * g4 + 1]), pack2bf(pv[4 * g4 + 2], pv[4 * g4 + 3])};    \
-      _Pragma("unroll") for (int dd = 0; dd < 4; ++dd) O[dd] *= alpha;                                     \
-      _Pragma("unroll") for (int kh = 0; kh < 2; ++kh) {                                                   \
-        /* selects, not pk[... + hl]: a lane-dependent index puts pk in scratch */                       \
-        const uint2 mine = hl ? pk[2 * kh + 1] : pk[2 * kh], give = hl ? pk[2 * kh] : pk[2 * kh + 1];      \
-        uint2 got;                                                                                         \
-        got.x = __shfl_xor(give.x, 32, WAVE);                                                              \
-        got.y = __shfl_xor(give.y, 32, WAVE);                                                              \
-        const v4u pb = hl == 0 ? v4u{mine.x, mine.y, got.x, got.y} : v4u{got.x, got.y, mine.x, mine.y};    \
-        _Pragma("unroll") for (int dd = 0; dd < 4; ++dd) {                                                 \
-          const v4u vf = __builtin_bit_cast(v4u, S.v[(32 * dd + kk) * 4 + 2 * kh + hl]);                  \
-          O[dd] = mfma32(vf, pb, O[dd]);                                                                   \
-        }                                                                                                  \
-      }                                                                                                    \
-    }                                                                                                      \
+  auto step = [&](const PfStage& S, int i) {
+    const int kb = t0 + 64 * i;
+    if (!(wact && kb <= w_hi && kb + 63 >= w_lo)) return;
+    f32x16 sc[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int x = 0; x < 16; ++x) sc[u][x] = 0.f;
+#pragma unroll
+    for (int h = 0; h < 8; ++h)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) sc[u] = mfma32(__builtin_bit_cast(v4u, S.k[u][h][lane]), qf[h], sc[u]);
+    if (!(wfull && kb >= w_full_lo && kb + 63 <= w_full_hi)) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int x = 0; x < 16; ++x) {
+          const int kx = kb + 32 * u + 16 * (x >> 3) + 8 * hl + (x & 7);
+          if (!(cvalid && kx >= lo_c && kx <= pos_c)) sc[u][x] = -INFINITY;
+        }
+    }
+    float mt = fmaxf(sc[0][0], sc[1][0]);
+#pragma unroll
+    for (int x = 1; x < 16; ++x) mt = fmaxf(mt, fmaxf(sc[0][x], sc[1][x]));
+    mt = fmaxf(mt, __shfl_xor(mt, 32, WAVE));
+    const float m_new = fmaxf(m_run, mt * scale_log2);
+    const float m_use = m_new == -INFINITY ? 0.f : m_new;  // no key yet: every term exp2(-inf) = 0
+    if (__any(m_new != m_run)) {
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+      l_run *= alpha;
+#pragma unroll
+      for (int dd = 0; dd < 4; ++dd) O[dd] *= alpha;
+      m_run = m_new;
+    }
+    float psum = 0.f;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int kh = 0; kh < 2; ++kh) {
+        float pv[8];
+#pragma unroll
+        for (int x = 0; x < 8; ++x) {
+          pv[x] = __builtin_amdgcn_exp2f(fmaf(sc[u][8 * kh + x], scale_log2, -m_use));
+          psum += pv[x];
+        }
+        const v4u pb = v4u{pack2bf(pv[0], pv[1]), pack2bf(pv[2], pv[3]), pack2bf(pv[4], pv[5]), pack2bf(pv[6], pv[7])};
+#pragma unroll
+        for (int dd = 0; dd < 4; ++dd)
+          O[dd] = mfma32(__builtin_bit_cast(v4u, S.v[u][2 * dd + kh][lane]), pb, O[dd]);
+      }
+    l_run += psum;
+  };
+  if (ntiles > 0) PF_ISSUE(st0, 0);  // (a row past the cache's end has no key to read)
+  for (int i = 0; i < nstep; i += 2) {
+    PF_SYNC();
+    PF_ISSUE(st1, i + 1);
+    step(st0, i);
+    if (i + 1 < nstep) {
+      PF_SYNC();
+      PF_ISSUE(st0, i + 2);
+      step(st1, i + 1);
+    }
   }
-  PF_ISSUE(st0, 0);
-  PF_ISSUE(st1, 1);
-  int t = 0;
-#define PF_STEP(SC, SI, t_)                                                                                \
-  {                                                                                                        \
-    PF_SYNC();                                                                                             \
-    PF_TILE(SC, t_);                                                                                       \
-    PF_ISSUE(SI, (t_) + 2);                                                                                \
-  }
-  for (; t + 2 < ntiles; t += 3) {
-    PF_STEP(st0, st2, t);
-    PF_STEP(st1, st0, t + 1);
-    PF_STEP(st2, st1, t + 2);
-  }
-  if (t < ntiles) PF_STEP(st0, st2, t);
-  if (t + 1 < ntiles) PF_STEP(st1, st0, t + 1);
-#undef PF_STEP
-#undef PF_TILE
 #undef PF_SYNC
 #undef PF_ISSUE
   __builtin_amdgcn_s_waitcnt(0);  // no direct load outlives the workgroup's LDS
@@ -760,10 +765,10 @@ __global__ __launch_bounds__(256) void k_attn_combine(const float* __restrict__ 
   T* yo = y + act_idx<T>(base + j, head * HD + d0, H * HD);
   if constexpr (sizeof(T) == 2) {
     uint4 pk;
-    pk.x = (uint32_t)f2bf(o[0] * inv) | ((uint32_t)f2bf(o[1] * inv) << 16);
-    pk.y = (uint32_t)f2bf(o[2] * inv) | ((uint32_t)f2bf(o[3] * inv) << 16);
-    pk.z = (uint32_t)f2bf(o[4] * inv) | ((uint32_t)f2bf(o[5] * inv) << 16);
-    pk.w = (uint32_t)f2bf(o[6] * inv) | ((uint32_t)f2bf(o[7] * inv) << 16);
+    pk.x = pack2bf(o[0] * inv, o[1] * inv);
+    pk.y = pack2bf(o[2] * inv, o[3] * inv);
+    pk.z = pack2bf(o[4] * inv, o[5] * inv);
+    pk.w = pack2bf(o[6] * inv, o[7] * inv);
     *(uint4*)yo = pk;
   } else {
 #pragma unroll
@@ -892,9 +897,10 @@ int fc_launch_attention(const void* q, const void* kc, const void* vc, void* y, 
     FC_CHECK_ARG(B * G <= 65535, "batch * n_kv_head must be <= 65535");
     const int ncolmax = max_per_row * (H / G);
     // prefill-width chunks: 128 query columns per workgroup, 32x32x16 MFMA
-    hipLaunchKernelGGL(k_attn_pf, dim3((ncolmax + 127) / 128, B * G), dim3(256), 0, s, (const bf16_t*)q,
+    const int nblk = (ncolmax + 127) / 128;
+    hipLaunchKernelGGL(k_attn_pf, dim3((unsigned)(8 * ((B * G + 7) / 8) * nblk)), dim3(256), 0, s, (const bf16_t*)q,
                        (const bf16_t*)kc, (const bf16_t*)vc, (bf16_t*)y, H, G, cap, row_off, start, max_per_row,
-                       max_tokens, window, scale * 1.4426950408889634f);
+                       max_tokens, window, scale * 1.4426950408889634f, B * G, nblk);
   } else if (dtype == FC_BF16 && hd == 128) {
     AttnGrid a = fc_attn_grid(B, max_per_row, typ_per_row, H, G, max_keys);
     const int64_t units = (int64_t)B * G * a.nqblk * a.nsplit * 16;

@@ -156,10 +156,10 @@ __global__ __launch_bounds__(256) void k_embed(const T* __restrict__ wte, const 
           const float ss = nred[j][0] + nred[j][1] + nred[j][2] + nred[j][3];
           const float inv = 1.f / sqrtf(ss / (float)D + 1e-6f);
           uint4 pk;
-          pk.x = (uint32_t)f2bf(keep[j][0] * inv) | ((uint32_t)f2bf(keep[j][1] * inv) << 16);
-          pk.y = (uint32_t)f2bf(keep[j][2] * inv) | ((uint32_t)f2bf(keep[j][3] * inv) << 16);
-          pk.z = (uint32_t)f2bf(keep[j][4] * inv) | ((uint32_t)f2bf(keep[j][5] * inv) << 16);
-          pk.w = (uint32_t)f2bf(keep[j][6] * inv) | ((uint32_t)f2bf(keep[j][7] * inv) << 16);
+          pk.x = pack2bf(keep[j][0] * inv, keep[j][1] * inv);
+          pk.y = pack2bf(keep[j][2] * inv, keep[j][3] * inv);
+          pk.z = pack2bf(keep[j][4] * inv, keep[j][5] * inv);
+          pk.w = pack2bf(keep[j][6] * inv, keep[j][7] * inv);
           *(uint4*)(h + frag_idx(base + j, c0, D)) = pk;  // 8 consecutive k: 16 contiguous bytes
         }
       }
@@ -479,8 +479,8 @@ __global__ __launch_bounds__(256) void k_rmsnorm(float* __restrict__ x, TO* __re
       const int64_t o = act_idx<TO>(row, 4 * i, D);
       if constexpr (sizeof(TO) == 2) {
         uint2 pk;
-        pk.x = (uint32_t)f2bf(v[u].x * inv) | ((uint32_t)f2bf(v[u].y * inv) << 16);
-        pk.y = (uint32_t)f2bf(v[u].z * inv) | ((uint32_t)f2bf(v[u].w * inv) << 16);
+        pk.x = pack2bf(v[u].x * inv, v[u].y * inv);
+        pk.y = pack2bf(v[u].z * inv, v[u].w * inv);
         *(uint2*)(h + o) = pk;
       } else {
         *(float4*)(h + o) = make_float4(v[u].x * inv, v[u].y * inv, v[u].z * inv, v[u].w * inv);

@@ -252,7 +252,7 @@ __device__ __forceinline__ void row_epilogue(const Epi& e, float (&v)[MT * NT / 
           o[c + 1] = a1;
           ss += a0 * a0 + a1 * a1;
           *(uint32_t*)(e.xa + frag_idx(m, n0 + col0 + c, (int)e.ldo)) =
-              (uint32_t)f2bf(a0) | ((uint32_t)f2bf(a1) << 16);
+              pack2bf(a0, a1);
         }
       }
 #pragma unroll
@@ -509,8 +509,8 @@ __device__ __forceinline__ void qkv_finish(const QkvEpi& Q, const float* x, int 
     uint32_t* w2 = (uint32_t*)&p2;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      w1[e] = (uint32_t)f2bf(x1[2 * e] * inv * 1.2f) | ((uint32_t)f2bf(x1[2 * e + 1] * inv * 1.2f) << 16);
-      w2[e] = (uint32_t)f2bf(x2[2 * e] * inv * 1.2f) | ((uint32_t)f2bf(x2[2 * e + 1] * inv * 1.2f) << 16);
+      w1[e] = pack2bf(x1[2 * e] * inv * 1.2f, x1[2 * e + 1] * inv * 1.2f);
+      w2[e] = pack2bf(x2[2 * e] * inv * 1.2f, x2[2 * e + 1] * inv * 1.2f);
     }
     if (hh < Q.H) {
       if (in_row) {
@@ -1490,7 +1490,7 @@ __global__ __launch_bounds__(256, MB == 2 ? 2 : 1) void k_gemm_big(
 #pragma unroll
           for (int hh = 0; hh < 2; ++hh) {
             const float x0 = fmaxf(acc[p][q][4 * j + 2 * hh], 0.f), x1 = fmaxf(acc[p][q][4 * j + 2 * hh + 1], 0.f);
-            pk[hh] = (uint32_t)f2bf(x0 * x0) | ((uint32_t)f2bf(x1 * x1) << 16);
+            pk[hh] = pack2bf(x0 * x0, x1 * x1);
           }
           *(uint2*)(scr + rl * 80 + (8 * j + ch) * 2) = uint2{pk[0], pk[1]};
         }
