@@ -66,7 +66,7 @@ class FcSpecState(Structure):
 
 
 EXPORTS = ["fc_last_error", "fc_version", "fc_forward_workspace_bytes", "fc_forward", "fc_gemm", "fc_pack_operand",
-           "fc_attention_workspace_bytes", "fc_attention", "fc_attention_noalloc", "fc_attention_noalloc_max_bytes",
+           "fc_attention_workspace_bytes", "fc_attention", "fc_attention_rows", "fc_attention_noalloc", "fc_attention_noalloc_max_bytes",
            "fc_attn_prologue", "fc_attn_qkv_workspace_bytes", "fc_attn_qkv", "fc_row_stats", "fc_row_stats_fields",
            "fc_spec_workspace_bytes",
            "fc_spec_round", "fc_spec_accept", "fc_spec_part_bytes", "fc_fast_sample", "fc_engine_sample",
@@ -93,6 +93,8 @@ def _declare(L):
     L.fc_attn_prologue.argtypes = [POINTER(FcModel), i32, POINTER(FcCache), vp, vp, vp, vp, vp, i32, vp, vp]
     L.fc_attention.argtypes = [vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, i32, vp, vp, i32, i32, i32, vp, i64,
                                vp]
+    L.fc_attention_rows.argtypes = L.fc_attention.argtypes
+    L.fc_attention_rows.restype = i32
     L.fc_attn_qkv_workspace_bytes.argtypes = [POINTER(FcModel), i32, i32]
     L.fc_attn_qkv_workspace_bytes.restype = i64
     L.fc_attn_qkv.argtypes = [POINTER(FcModel), i32, POINTER(FcCache), vp, vp, vp, vp, i32, i32, vp, vp, i64, vp]

@@ -176,6 +176,12 @@ __device__ __forceinline__ f32x4 mfma16a(uint4 a, uint4 b, f32x4 c) {
                                                   0, 0);
 }
 
+// Where the attention kernels put 8 consecutive values (dims d .. +7 of a
+// head) of token m: c_proj's operand order, or row-major (`rows`).
+__device__ __forceinline__ int64_t y_idx(int64_t m, int k, int K, int rows) {
+  return rows ? m * K + k : frag_idx(m, k, K);
+}
+
 // One 32-key tile of one wave: scores S^T = K Q^T, online softmax update,
 // O^T += V^T P^T (see the kernel comment).
 __device__ __forceinline__ void attn_tile(const uint4 (&kf)[2][4], const uint4 (&vf)[8], const uint4 (&qf)[4],
@@ -237,7 +243,7 @@ __global__ __launch_bounds__(64 * NW) void k_attn_mfma(const bf16_t* __restrict_
                                                        int G, int cap, const int* __restrict__ row_off,
                                                        const int* __restrict__ start, int max_per_row, int Mcap,
                                                        int window, int split_keys, int nsplit, int nqblk,
-                                                       float scale_log2) {
+                                                       float scale_log2, int rows) {
   constexpr int HD = 128;
   const int split = blockIdx.x, bg = blockIdx.y, qb = blockIdx.z;
   const int b = bg / G, g = bg - b * G, rep = H / G;
@@ -351,7 +357,7 @@ __global__ __launch_bounds__(64 * NW) void k_attn_mfma(const bf16_t* __restrict_
     pk.y = pack2bf(o[2] * inv, o[3] * inv);
     pk.z = pack2bf(o[4] * inv, o[5] * inv);
     pk.w = pack2bf(o[6] * inv, o[7] * inv);
-    *(uint4*)(y + frag_idx(base + jq, hq * HD + d0, H * HD)) = pk;
+    *(uint4*)(y + y_idx(base + jq, hq * HD + d0, H * HD, rows)) = pk;
     return;
   }
   float4* po = (float4*)(part_o + (pidx * 16 + qc) * HD + d0);
@@ -375,7 +381,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn_mfma_qb(const bf16_t* __res
                                                        int G, int cap, const int* __restrict__ row_off,
                                                        const int* __restrict__ start, int max_per_row, int Mcap,
                                                        int window, int split_keys, int nsplit, int nqblk,
-                                                       float scale_log2) {
+                                                       float scale_log2, int rows) {
   constexpr int HD = 128;
   const int split = blockIdx.x, bg = blockIdx.y, qb0 = blockIdx.z * QB;
   const int b = bg / G, g = bg - b * G, rep = H / G;
@@ -515,7 +521,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn_mfma_qb(const bf16_t* __res
             pk.y = pack2bf(o[2] * inv, o[3] * inv);
             pk.z = pack2bf(o[4] * inv, o[5] * inv);
             pk.w = pack2bf(o[6] * inv, o[7] * inv);
-            *(uint4*)(y + frag_idx(base + jq, hq * HD + d0, H * HD)) = pk;
+            *(uint4*)(y + y_idx(base + jq, hq * HD + d0, H * HD, rows)) = pk;
           }
         } else {
           float4* po = (float4*)(part_o + (pidx * 16 + qc) * HD + d0);
@@ -549,23 +555,33 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn_mfma_qb(const bf16_t* __res
 //
 // What bounds it: per 32 keys x 32 columns 512 MFMA cycles against ~540 VALU
 // (256 of them the exponentials), overlapped by the two waves of a SIMD; hence
-// the output is rescaled only in steps that raise some column's maximum.
+// the output is rescaled only where some column's maximum has risen by more
+// than PF_SLACK binary orders over the one in use (terms reach 2^PF_SLACK then,
+// the same relative rounding in bf16 and fp32).
 // 8 rows x 500-1000 queries, 12 heads, window 1024: 112 -> 70 us (before: 32 keys
 // per barrier, operands in the caches' order, an exchange per P operand).
 //
 // Workgroups: all column blocks of a (row, group) on one XCD (its K and V in
 // one L2), the last blocks, which see the most keys, first.
+#define PF_SLACK 8.f
 struct PfStage {
   uint4 k[2][8][64];  // [32-key tile][16-dim slice][lane]
   uint4 v[2][8][64];  // [32-key tile][2 (dim / 32) + key half][lane]
 };
-__global__ __launch_bounds__(256, 2) void k_attn_pf(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
+// KS = 2: eight waves, the second four taking every other step of the same
+// columns with stages of their own, the halves merged in LDS at the end. For
+// launches of at most one workgroup per CU, where a wave otherwise has its
+// SIMD to itself and walks all keys (4 x 476 queries on 1024-1500 keys, 6
+// heads, 96 workgroups: 38 -> 31 us; at 384 workgroups one group is the faster,
+// 30 against 39).
+template <int KS>
+__global__ __launch_bounds__(256 * KS, 2) void k_attn_pf(const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc,
                                                  const bf16_t* __restrict__ vc, bf16_t* __restrict__ y, int H, int G,
                                                  int cap, const int* __restrict__ row_off,
                                                  const int* __restrict__ start, int max_per_row, int Mcap,
-                                                 int window, float scale_log2, int nbg, int nblk) {
+                                                 int window, float scale_log2, int nbg, int nblk, int rows) {
   constexpr int HD = 128;
-  __shared__ PfStage st0, st1;
+  __shared__ PfStage stg0[KS], stg1[KS];
   const int nbgl = (nbg + 7) >> 3, jj = blockIdx.x >> 3;
   const int bg = (jj % nbgl) * 8 + (blockIdx.x & 7);
   if (bg >= nbg) return;
@@ -575,14 +591,15 @@ __global__ __launch_bounds__(256, 2) void k_attn_pf(const bf16_t* __restrict__ q
   const int ncol = n * rep;
   const int c0 = (nblk - 1 - jj / nbgl) * 128;
   if (c0 >= ncol) return;  // the whole workgroup
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wid & 3, grp = KS > 1 ? wid >> 2 : 0;
   const int hl = lane >> 5, kk = lane & 31;
   // the workgroup's key range
   const int lcol = min(c0 + 127, ncol - 1);
   const int kbeg = window > 0 ? max(0, s0 + c0 / rep - window) : 0;
   const int kend = min(s0 + lcol / rep + 1, cap);
   const int t0 = kbeg & ~31;
-  const int ntiles = (kend - t0 + 31) >> 5, nstep = (ntiles + 1) >> 1;
+  const int ntiles = (kend - t0 + 31) >> 5, nstep = (ntiles + 1) >> 1;  // group grp takes steps grp, grp + KS, ..
   // this wave's columns and key range
   const int wc0 = c0 + 32 * wave;
   const bool wact = wc0 < ncol;
@@ -652,10 +669,25 @@ __global__ __launch_bounds__(256, 2) void k_attn_pf(const bf16_t* __restrict__ q
     for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int x = 0; x < 16; ++x) sc[u][x] = 0.f;
+    // all K operands are read ahead of the first product, V's behind the last
+    // one and ahead of the softmax (read one or two ahead of their use, as the
+    // compiler places them, each product waits out an LDS latency)
+    v4u kf[8][2], vf[2][8];
 #pragma unroll
     for (int h = 0; h < 8; ++h)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) sc[u] = mfma32(__builtin_bit_cast(v4u, S.k[u][h][lane]), qf[h], sc[u]);
+      for (int u = 0; u < 2; ++u) kf[h][u] = __builtin_bit_cast(v4u, S.k[u][h][lane]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int h = 0; h < 8; ++h)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) sc[u] = mfma32(kf[h][u], qf[h], sc[u]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int f = 0; f < 8; ++f) vf[u][f] = __builtin_bit_cast(v4u, S.v[u][f][lane]);
+    __builtin_amdgcn_sched_barrier(0);
     if (!(wfull && kb >= w_full_lo && kb + 63 <= w_full_hi)) {
 #pragma unroll
       for (int u = 0; u < 2; ++u)
@@ -665,20 +697,26 @@ __global__ __launch_bounds__(256, 2) void k_attn_pf(const bf16_t* __restrict__ q
           if (!(cvalid && kx >= lo_c && kx <= pos_c)) sc[u][x] = -INFINITY;
         }
     }
-    float mt = fmaxf(sc[0][0], sc[1][0]);
+    float m4[4];  // four chains each: one or two waves per SIMD leave latencies in sight
 #pragma unroll
-    for (int x = 1; x < 16; ++x) mt = fmaxf(mt, fmaxf(sc[0][x], sc[1][x]));
-    mt = fmaxf(mt, __shfl_xor(mt, 32, WAVE));
+    for (int x = 0; x < 4; ++x) m4[x] = fmaxf(sc[0][x], sc[1][x]);
+#pragma unroll
+    for (int x = 4; x < 16; ++x) m4[x & 3] = fmaxf(m4[x & 3], fmaxf(sc[0][x], sc[1][x]));
+    float mt = fmaxf(fmaxf(m4[0], m4[1]), fmaxf(m4[2], m4[3]));
+    {
+      const auto h2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(mt), __float_as_uint(mt), false, false);
+      mt = fmaxf(__uint_as_float(h2[0]), __uint_as_float(h2[1]));  // lanes l and l ^ 32: the column's two key halves
+    }
     const float m_new = fmaxf(m_run, mt * scale_log2);
-    const float m_use = m_new == -INFINITY ? 0.f : m_new;  // no key yet: every term exp2(-inf) = 0
-    if (__any(m_new != m_run)) {
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+    if (__any(m_new > m_run + PF_SLACK)) {
+      const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.f : m_new));
       l_run *= alpha;
 #pragma unroll
       for (int dd = 0; dd < 4; ++dd) O[dd] *= alpha;
       m_run = m_new;
     }
-    float psum = 0.f;
+    const float m_use = m_run == -INFINITY ? 0.f : m_run;  // no key yet: every term exp2(-inf) = 0
+    float ps[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -687,33 +725,64 @@ __global__ __launch_bounds__(256, 2) void k_attn_pf(const bf16_t* __restrict__ q
 #pragma unroll
         for (int x = 0; x < 8; ++x) {
           pv[x] = __builtin_amdgcn_exp2f(fmaf(sc[u][8 * kh + x], scale_log2, -m_use));
-          psum += pv[x];
+          ps[x & 3] += pv[x];
         }
         const v4u pb = v4u{pack2bf(pv[0], pv[1]), pack2bf(pv[2], pv[3]), pack2bf(pv[4], pv[5]), pack2bf(pv[6], pv[7])};
 #pragma unroll
         for (int dd = 0; dd < 4; ++dd)
-          O[dd] = mfma32(__builtin_bit_cast(v4u, S.v[u][2 * dd + kh][lane]), pb, O[dd]);
+          O[dd] = mfma32(vf[u][2 * dd + kh], pb, O[dd]);
       }
-    l_run += psum;
+    l_run += (ps[0] + ps[1]) + (ps[2] + ps[3]);
   };
-  if (ntiles > 0) PF_ISSUE(st0, 0);  // (a row past the cache's end has no key to read)
-  for (int i = 0; i < nstep; i += 2) {
+  if (ntiles > 0) PF_ISSUE(stg0[grp], grp);  // (a row past the cache's end has no key to read)
+  for (int i = 0; i < nstep; i += 2 * KS) {
     PF_SYNC();
-    PF_ISSUE(st1, i + 1);
-    step(st0, i);
-    if (i + 1 < nstep) {
+    PF_ISSUE(stg1[grp], i + KS + grp);
+    step(stg0[grp], i + grp);
+    if (i + KS < nstep) {
       PF_SYNC();
-      PF_ISSUE(st0, i + 2);
-      step(st1, i + 1);
+      PF_ISSUE(stg0[grp], i + 2 * KS + grp);
+      step(stg1[grp], i + KS + grp);
     }
   }
 #undef PF_SYNC
 #undef PF_ISSUE
-  __builtin_amdgcn_s_waitcnt(0);  // no direct load outlives the workgroup's LDS
-  if (!cvalid) return;
+  __builtin_amdgcn_s_waitcnt(0);  // no direct load outlives its stage
+  __syncthreads();                // the stages become scratch
+  if constexpr (KS == 2) {
+    // the second group's O, maximum and sum, lane for lane
+    float(*xo)[64][64] = (float(*)[64][64])&stg0[0];  // [wave][value][lane], 64 KB
+    float(*xm)[2][64] = (float(*)[2][64])&stg1[0];
+    static_assert(sizeof(stg0) >= 4 * 64 * 64 * 4, "the second group's output");
+    if (grp == 1) {
+#pragma unroll
+      for (int dd = 0; dd < 4; ++dd)
+#pragma unroll
+        for (int x = 0; x < 16; ++x) xo[wave][16 * dd + x][lane] = O[dd][x];
+      xm[wave][0][lane] = m_run;
+      xm[wave][1][lane] = l_run;
+    }
+    __syncthreads();
+    if (grp == 0) {
+      const float m1 = xm[wave][0][lane], m = fmaxf(m_run, m1), mu = m == -INFINITY ? 0.f : m;
+      const float a0 = __builtin_amdgcn_exp2f(m_run - mu), a1 = __builtin_amdgcn_exp2f(m1 - mu);
+      l_run = l_run * a0 + xm[wave][1][lane] * a1;
+#pragma unroll
+      for (int dd = 0; dd < 4; ++dd)
+#pragma unroll
+        for (int x = 0; x < 16; ++x) O[dd][x] = O[dd][x] * a0 + xo[wave][16 * dd + x][lane] * a1;
+    }
+    __syncthreads();
+    if (grp == 1) return;
+  }
   const float l_tot = l_run + __shfl_xor(l_run, 32, WAVE);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  // lane: column l % 32; register 4 i4 + x of O[dd] is dim 32 dd + 8 i4 + 4 hl + x
+  // lane: column l % 32; register 4 i4 + x of O[dd] is dim 32 dd + 8 i4 + 4 hl + x.
+  // Through LDS (rows of 136 values) so that a lane writes 8 dims of a column:
+  // 16 columns x 4 groups per store in operand order (1 KB in a row where the
+  // columns are 16 tokens), 4 columns of 256 bytes in row-major order.
+  bf16_t* T = (bf16_t*)(wave < 2 ? &stg0[0] : &stg1[0]) + (wave & 1) * 32 * 136;
+  static_assert(sizeof(PfStage) >= 2 * 32 * 136 * 2, "two waves' scratch");
 #pragma unroll
   for (int dd = 0; dd < 4; ++dd)
 #pragma unroll
@@ -721,8 +790,17 @@ __global__ __launch_bounds__(256, 2) void k_attn_pf(const bf16_t* __restrict__ q
       uint2 pk;
       pk.x = pack2bf(O[dd][4 * i4] * inv, O[dd][4 * i4 + 1] * inv);
       pk.y = pack2bf(O[dd][4 * i4 + 2] * inv, O[dd][4 * i4 + 3] * inv);
-      *(uint2*)(y + frag_idx(base + j, head * HD + 32 * dd + 8 * i4 + 4 * hl, H * HD)) = pk;
+      *(uint2*)(T + kk * 136 + 32 * dd + 8 * i4 + 4 * hl) = pk;
     }
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int it = 0; it < 8; ++it) {
+    const int cc = rows ? 4 * it + (lane >> 4) : (lane & 15) + 16 * (it & 1);
+    const int d0 = 8 * (rows ? lane & 15 : (lane >> 4) + 4 * (it >> 1));
+    const uint4 val = *(const uint4*)(T + cc * 136 + d0);
+    const int co = wc0 + cc, jo = co / rep;
+    if (co < ncol) *(uint4*)(y + y_idx(base + jo, (g * rep + co - jo * rep) * HD + d0, H * HD, rows)) = val;
+  }
 }
 
 // One workgroup per (row, KV group, query block): merge the key splits of
@@ -732,7 +810,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_attn_combine(const float* __restrict__ part_o,
                                                       const float* __restrict__ part_ml, T* __restrict__ y, int H,
                                                       int G, int nqblk, int nsplit, const int* __restrict__ row_off,
-                                                      int max_per_row, int Mcap) {
+                                                      int max_per_row, int Mcap, int rows) {
   constexpr int HD = 128;
   const int bg = blockIdx.x, qb = blockIdx.y;
   const int b = bg / G, g = bg - b * G, rep = H / G;
@@ -762,7 +840,8 @@ __global__ __launch_bounds__(256) void k_attn_combine(const float* __restrict__ 
   const float inv = L > 0.f ? 1.f / L : 0.f;
   // y is the c_proj GEMM's operand [token][H * 128]: 8 consecutive k are one
   // contiguous 16-byte group in both layouts
-  T* yo = y + act_idx<T>(base + j, head * HD + d0, H * HD);
+  T* yo = y + (sizeof(T) == 2 ? y_idx(base + j, head * HD + d0, H * HD, rows)
+                              : (int64_t)(base + j) * H * HD + head * HD + d0);
   if constexpr (sizeof(T) == 2) {
     uint4 pk;
     pk.x = pack2bf(o[0] * inv, o[1] * inv);
@@ -785,7 +864,7 @@ __global__ __launch_bounds__(256) void k_attn_valu(const T* __restrict__ q, cons
                                                    const T* __restrict__ vc, T* __restrict__ y, int H, int G, int hd,
                                                    int cap, const int* __restrict__ row_off,
                                                    const int* __restrict__ start, int max_per_row, int Mcap,
-                                                   int window, float scale) {
+                                                   int window, float scale, int rows) {
   __shared__ float qs[128];
   __shared__ float sc[VALU_MAXK];
   __shared__ float red[16];
@@ -827,7 +906,7 @@ __global__ __launch_bounds__(256) void k_attn_valu(const T* __restrict__ q, cons
       const int key = lo + i;
       acc += sc[i] * ld<T>(vb, ((int64_t)(key >> 5) * hd + d) * 32 + (key & 31));
     }
-    st<T>(y, act_idx<T>(m, h * hd + d, H * hd), acc);
+    st<T>(y, sizeof(T) == 2 ? y_idx(m, h * hd + d, H * hd, rows) : (int64_t)m * H * hd + h * hd + d, acc);
   }
 }
 
@@ -888,7 +967,7 @@ static bool attn_uses_pf(int dtype, int hd, int typ_per_row, int H, int G) {
 int fc_launch_attention(const void* q, const void* kc, const void* vc, void* y, int B, int max_tokens,
                         int max_per_row, int typ_per_row, int H, int G, int hd, int cap, const int* row_off,
                         const int* start, int window, int max_keys, int dtype, void* part, int64_t part_bytes,
-                        hipStream_t s) {
+                        hipStream_t s, int rows) {
   FC_CHECK_ARG(H % G == 0, "n_head must be a multiple of n_kv_head");
   FC_CHECK_ARG(cap % 32 == 0, "cache capacity must be a multiple of 32");
   FC_CHECK_ARG(max_per_row > 0, "max_per_row");
@@ -898,9 +977,16 @@ int fc_launch_attention(const void* q, const void* kc, const void* vc, void* y, 
     const int ncolmax = max_per_row * (H / G);
     // prefill-width chunks: 128 query columns per workgroup, 32x32x16 MFMA
     const int nblk = (ncolmax + 127) / 128;
-    hipLaunchKernelGGL(k_attn_pf, dim3((unsigned)(8 * ((B * G + 7) / 8) * nblk)), dim3(256), 0, s, (const bf16_t*)q,
-                       (const bf16_t*)kc, (const bf16_t*)vc, (bf16_t*)y, H, G, cap, row_off, start, max_per_row,
-                       max_tokens, window, scale * 1.4426950408889634f, B * G, nblk);
+    const dim3 grid((unsigned)(8 * ((B * G + 7) / 8) * nblk));
+    const float sl2 = scale * 1.4426950408889634f;
+    // two key halves per workgroup up to about one workgroup per CU (272
+    // workgroups: 50 -> 40 us, 384: 30 -> 39)
+    if ((int64_t)B * G * nblk <= 288 && max_keys >= 256)
+      hipLaunchKernelGGL(k_attn_pf<2>, grid, dim3(512), 0, s, (const bf16_t*)q, (const bf16_t*)kc, (const bf16_t*)vc,
+                         (bf16_t*)y, H, G, cap, row_off, start, max_per_row, max_tokens, window, sl2, B * G, nblk, rows);
+    else
+      hipLaunchKernelGGL(k_attn_pf<1>, grid, dim3(256), 0, s, (const bf16_t*)q, (const bf16_t*)kc, (const bf16_t*)vc,
+                         (bf16_t*)y, H, G, cap, row_off, start, max_per_row, max_tokens, window, sl2, B * G, nblk, rows);
   } else if (dtype == FC_BF16 && hd == 128) {
     AttnGrid a = fc_attn_grid(B, max_per_row, typ_per_row, H, G, max_keys);
     const int64_t units = (int64_t)B * G * a.nqblk * a.nsplit * 16;
@@ -914,15 +1000,15 @@ int fc_launch_attention(const void* q, const void* kc, const void* vc, void* y, 
       hipLaunchKernelGGL((k_attn_mfma_qb<FC_ATTN_WAVES, 2>), dim3(a.nsplit, B * G, (a.nqblk + 1) / 2),
                          dim3(64 * FC_ATTN_WAVES), 0, s, (const bf16_t*)q, (const bf16_t*)kc, (const bf16_t*)vc, po,
                          pml, (bf16_t*)y, H, G, cap, row_off, start, max_per_row, max_tokens, window, a.split_keys,
-                         a.nsplit, a.nqblk, sl2);
+                         a.nsplit, a.nqblk, sl2, rows);
     else
       hipLaunchKernelGGL(k_attn_mfma<FC_ATTN_WAVES>, dim3(a.nsplit, B * G, a.nqblk), dim3(64 * FC_ATTN_WAVES),
                          0, s, (const bf16_t*)q, (const bf16_t*)kc, (const bf16_t*)vc, po, pml, (bf16_t*)y, H, G, cap,
-                         row_off, start, max_per_row, max_tokens, window, a.split_keys, a.nsplit, a.nqblk, sl2);
+                         row_off, start, max_per_row, max_tokens, window, a.split_keys, a.nsplit, a.nqblk, sl2, rows);
     if (a.nsplit > 1) {
       FC_LAUNCH_CHECK();
       hipLaunchKernelGGL(k_attn_combine<bf16_t>, dim3(B * G, a.nqblk), dim3(256), 0, s, po, pml, (bf16_t*)y, H, G,
-                         a.nqblk, a.nsplit, row_off, max_per_row, max_tokens);
+                         a.nqblk, a.nsplit, row_off, max_per_row, max_tokens, rows);
     }
   } else {
     FC_CHECK_ARG(hd <= 128, "head_dim must be <= 128");
@@ -931,11 +1017,11 @@ int fc_launch_attention(const void* q, const void* kc, const void* vc, void* y, 
     if (dtype == FC_BF16)
       hipLaunchKernelGGL(k_attn_valu<bf16_t>, grid, dim3(256), 0, s, (const bf16_t*)q, (const bf16_t*)kc,
                          (const bf16_t*)vc, (bf16_t*)y, H, G, hd, cap, row_off, start, max_per_row, max_tokens,
-                         window, scale);
+                         window, scale, rows);
     else
       hipLaunchKernelGGL(k_attn_valu<float>, grid, dim3(256), 0, s, (const float*)q, (const float*)kc,
                          (const float*)vc, (float*)y, H, G, hd, cap, row_off, start, max_per_row, max_tokens, window,
-                         scale);
+                         scale, rows);
   }
   FC_LAUNCH_CHECK();
   return FC_OK;
@@ -955,7 +1041,19 @@ extern "C" int32_t fc_attention(const void* q, const void* kc, const void* vc, v
   FC_CHECK_ARG(batch > 0 && max_tokens > 0 && max_per_row > 0 && n_head > 0 && n_kv_head > 0, "sizes");
   FC_CHECK_ARG(max_keys > 0 && max_keys <= cap, "max_keys must be in [1, cap]");
   return fc_launch_attention(q, kc, vc, y, batch, max_tokens, max_per_row, max_per_row, n_head, n_kv_head, head_dim,
-                             cap, row_off, start, window, max_keys, dtype, work, work_bytes, (hipStream_t)stream);
+                             cap, row_off, start, window, max_keys, dtype, work, work_bytes, (hipStream_t)stream, 0);
+}
+
+extern "C" int32_t fc_attention_rows(const void* q, const void* kc, const void* vc, void* y, int32_t batch,
+                                     int32_t max_tokens, int32_t max_per_row, int32_t n_head, int32_t n_kv_head,
+                                     int32_t head_dim, int32_t cap, const int32_t* row_off, const int32_t* start,
+                                     int32_t window, int32_t max_keys, int32_t dtype, void* work, int64_t work_bytes,
+                                     void* stream) {
+  FC_CHECK_ARG(q && kc && vc && y && row_off && start, "null pointer");
+  FC_CHECK_ARG(batch > 0 && max_tokens > 0 && max_per_row > 0 && n_head > 0 && n_kv_head > 0, "sizes");
+  FC_CHECK_ARG(max_keys > 0 && max_keys <= cap, "max_keys must be in [1, cap]");
+  return fc_launch_attention(q, kc, vc, y, batch, max_tokens, max_per_row, max_per_row, n_head, n_kv_head, head_dim,
+                             cap, row_off, start, window, max_keys, dtype, work, work_bytes, (hipStream_t)stream, 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -1044,5 +1142,5 @@ extern "C" int32_t fc_attention_noalloc(const void* q, const void* kc, const voi
   if (rc != FC_OK) return rc;
   return fc_launch_attention(q, kc, vc, y, batch, max_tokens, max_per_row, max_per_row, n_head, n_kv_head, head_dim,
                              cap, row_off, start, window, max_keys, dtype, part, FC_NOALLOC_SCRATCH_BYTES,
-                             (hipStream_t)stream);
+                             (hipStream_t)stream, 0);
 }

@@ -130,7 +130,7 @@ int64_t fc_attn_part_bytes(int batch, int max_per_row, int n_head, int n_kv_head
 int fc_launch_attention(const void* q, const void* kc, const void* vc, void* y, int B, int max_tokens,
                         int max_per_row, int typ_per_row, int H, int G, int hd, int cap, const int* row_off,
                         const int* start, int window, int max_keys, int dtype, void* part, int64_t part_bytes,
-                        hipStream_t s);
+                        hipStream_t s, int rows = 0);  // rows: bf16 y row-major instead of c_proj's operand order
 // fc_attention_noalloc's scratch address for the stream's GPU, looked up now
 // (fc_graph_begin runs it before a capture starts)
 int fc_noalloc_prepare(hipStream_t stream);

@@ -143,14 +143,11 @@ def attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, row
     max_keys = min(cap, window + max_per_row) if window > 0 else cap
     nb = lib().fc_attention_workspace_bytes(B, max_per_row, H, G, hd, max_keys)
     ws = torch.empty(max(nb, 1), dtype=torch.uint8, device=q.device)
-    rows = (tot + 15) // 16 * 16 if code == _lib.FC_BF16 else tot
-    y = torch.empty((max(rows, 1), H * hd), dtype=q.dtype, device=q.device)
+    y = torch.empty((max(tot, 1), H * hd), dtype=q.dtype, device=q.device)
     qc = q.contiguous()
-    check(lib().fc_attention(qc.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), y.data_ptr(), B, tot,
+    check(lib().fc_attention_rows(qc.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), y.data_ptr(), B, tot,
                              max_per_row, H, G, hd, cap, row_off.data_ptr(), start.data_ptr(), window, max_keys,
-                             code, ws.data_ptr(), ws.numel(), _stream(q)), "fc_attention")
-    if code == _lib.FC_BF16:
-        return frag_to_rows(y, tot).contiguous()
+                             code, ws.data_ptr(), ws.numel(), _stream(q)), "fc_attention_rows")
     return y[:tot]
 
 

@@ -215,6 +215,12 @@ int32_t fc_attention(const void* q, const void* kc, const void* vc, void* y,
                      const int32_t* start, int32_t window, int32_t max_keys, int32_t dtype, void* work,
                      int64_t work_bytes, void* stream);
 
+/* fc_attention with y row-major ([max_tokens][H*hd]) in bf16 as well. */
+int32_t fc_attention_rows(const void* q, const void* kc, const void* vc, void* y, int32_t batch, int32_t max_tokens,
+                          int32_t max_per_row, int32_t n_head, int32_t n_kv_head, int32_t head_dim, int32_t cap,
+                          const int32_t* row_off, const int32_t* start, int32_t window, int32_t max_keys,
+                          int32_t dtype, void* work, int64_t work_bytes, void* stream);
+
 /* fc_attention without the workspace argument: the split-KV partials live in
  * a static device array of the library, fc_attention_noalloc_max_bytes()
  * bytes (32 MiB), which each GPU the library runs on holds until the process
