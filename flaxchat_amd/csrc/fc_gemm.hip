@@ -8,7 +8,8 @@
 // (engine.py:164-166) and the 15*tanh(z/15) softcap (engine.py:173-174).
 //
 // Kernels:
-//   k_gemv     VALU dot products (fp32 weights: the parity mode).
+//   k_gemv     VALU dot products (fp32 weights, the parity mode, up to 8 rows).
+//   k_gemm_f32 fp32 MFMA, 64 x 64 or K-split 32 x 32 tiles (fp32, more rows).
 //   k_gemm_ks  bf16 MFMA 16x16x32, workgroup tile of 16-32 rows x 16-64
 //              columns, the four waves split K, register pipeline; draft
 //              steps and the split-K residual GEMMs.
@@ -183,6 +184,162 @@ __global__ __launch_bounds__(256) void k_gemv(const T* __restrict__ A, const T* 
 #pragma unroll
     for (int c = 0; c < 4; ++c)
       if (lane == ((i * 4 + c) & 63) && m0 + i < M && n0 + c < N) epi_apply<EPI>(e, m0 + i, n0 + c, acc[i][c]);
+}
+
+// ---------------------------------------------------------------------------
+// fp32 GEMM on the fp32 matrix cores (32x32x2: true fp32 products and sums at
+// twice the rate of unpacked VALU FMAs), for more than GEMV_MAX_M rows.
+//
+// KW = 1: a workgroup owns 64 x 64 outputs, its 2 x 2 waves 32 x 32 each;
+// KW = 4, 8: 32 x 32 outputs, the KW waves take every KW-th 32-deep k chunk
+// and are summed in LDS (outputs too few for 64 x 64 tiles to fill the CUs).
+// A chunk's rows (128 bytes of 32 rows per operand) go to LDS by direct loads,
+// whole lines, two stages. Lane l takes its operands 16 bytes at a time: row
+// l % 32, k 8 j + 4 (l / 32) .. +3, whose component x is MFMA x of group j (the
+// order of k within a chunk is free). For that the 16-byte piece p of row r
+// lies at place p ^ (r % 8), so that eight rows' pieces do not share banks.
+//
+// Rounding: a group of 8 k is summed from zero, four groups pairwise, and the
+// chunks with TwoSum (the error terms in a second accumulator), so the error
+// does not grow with K: against 64 bits 7.1e-8 at K = 256 and 3072 where k_gemv,
+// whose lanes sum K / 64 products each, has 7.8e-8 and 1.4e-7. Row-major
+// operands, K % 8 == 0.
+//
+// 1000 rows x 8192 x 256: 493 -> 63 us, x 1024 x 256: 68 -> 13.7, x 256 x 1024:
+// 32 -> 12.7 (k_gemv re-reads the weights every 8 rows and does 4 FMAs per
+// load). Bound by the MFMAs (1024 cycles a chunk) and, not overlapped with them
+// within a wave, the 16 x 10 VALU operations of its sums.
+// ---------------------------------------------------------------------------
+#define GEMV_MAX_M 16
+__device__ __forceinline__ f32x16 mfma32f(float a, float b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+struct F32Stage {
+  float4 a[32][8], w[32][8];  // 32 rows x 32 k per operand, pieces swizzled
+};
+// TwoSum: tot + low += t, exactly in tot and its error term (NaN once tot is infinite: f32_round2)
+__device__ __forceinline__ void f32_add2(float& tot, float& low, float t) {
+  const float s = tot + t, b = s - tot;
+  low += (tot - (s - b)) + (t - b);
+  tot = s;
+}
+__device__ __forceinline__ float f32_round2(float tot, float low) {
+  return fabsf(tot) < INFINITY ? tot + low : tot;
+}
+template <int KW, int EPI>
+__global__ __launch_bounds__(KW == 8 ? 512 : 256, 2) void k_gemm_f32(const float* __restrict__ A, const float* __restrict__ W,
+                                                     int Mcap, const int* __restrict__ Mdev, int N, int K, int ntiles,
+                                                     Epi e) {
+  constexpr int T = KW == 1 ? 64 : 32;
+  // KW = 1: a row half of A and W each; else a wave each
+  __shared__ F32Stage st0[KW == 1 ? 2 : KW], st1[KW == 1 ? 2 : KW];
+  const int M = Mdev ? min(*Mdev, Mcap) : Mcap;
+  const int nt = blockIdx.x % ntiles, mt = blockIdx.x / ntiles;
+  const int m0 = mt * T, n0 = nt * T;
+  if (m0 >= M) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = KW == 1 ? wave >> 1 : 0, wn = KW == 1 ? wave & 1 : 0;
+  const int C = (K + 31) >> 5;                              // chunks; a wave takes chunks wave, wave + KW, ...
+  const int nch = (C + KW - 1) / KW;
+  // direct loads: lane l fetches the piece that lies at place l % 8 of row
+  // l / 8 of a group of eight rows. KW = 1: wave w loads operand w / 2's half
+  // w % 2 (rows 32 (w % 2) .. +31); KW > 1: both operands of its own chunk
+  const int lr = lane >> 3, lp = (lane & 7) ^ lr;
+  auto issue = [&](F32Stage* st, int ci) {
+    const int c = min(KW == 1 ? ci : KW * ci + wave, C - 1);  // past the end: harmless re-reads
+    const uint32_t koff = (uint32_t)min(32 * c + 4 * lp, K - 4) * 4u;    // past the row's end: its last piece again
+    auto rows = [&](const float* P, int r0, int R, uint32_t lds) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {  // rows r0 + 8 u .. +7, clamped to the last one
+        const uint32_t row = (uint32_t)min(8 * u + lr, R - 1 - r0);
+        lds_load_1k(P + (int64_t)r0 * K, row * (uint32_t)K * 4u + koff, lds + 1024 * u);
+      }
+    };
+    if constexpr (KW == 1) {
+      const int h = wave & 1;
+      if (wave < 2) rows(A, min(m0 + 32 * h, M - 1), M, LDS_ADDR(st[0].a) + (uint32_t)sizeof(F32Stage) * h);
+      else rows(W, min(n0 + 32 * h, N - 1), N, LDS_ADDR(st[0].w) + (uint32_t)sizeof(F32Stage) * h);
+    } else {
+      rows(A, m0, M, LDS_ADDR(st[0].a) + (uint32_t)sizeof(F32Stage) * wave);
+      rows(W, n0, N, LDS_ADDR(st[0].w) + (uint32_t)sizeof(F32Stage) * wave);
+    }
+  };
+  float tot[16], low[16];
+#pragma unroll
+  for (int x = 0; x < 16; ++x) tot[x] = low[x] = 0.f;
+  const int r = lane & 31, hl = lane >> 5;
+  auto chunk = [&](const F32Stage* st, int ci) {
+    const int c = KW == 1 ? ci : KW * ci + wave;
+    if (c >= C) return;
+    const F32Stage& sa = st[KW == 1 ? wm : wave];
+    const F32Stage& sw = st[KW == 1 ? wn : wave];
+    const int jn = min(4, (K - 32 * c) >> 3);  // groups of 8 k in the chunk
+    f32x16 g[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+      for (int x = 0; x < 16; ++x) g[j][x] = 0.f;
+      if (j < jn) {
+        const float4 av = sa.a[r][(2 * j + hl) ^ (r & 7)], wv = sw.w[r][(2 * j + hl) ^ (r & 7)];
+        g[j] = mfma32f(av.x, wv.x, g[j]);
+        g[j] = mfma32f(av.y, wv.y, g[j]);
+        g[j] = mfma32f(av.z, wv.z, g[j]);
+        g[j] = mfma32f(av.w, wv.w, g[j]);
+      }
+    }
+#pragma unroll
+    for (int x = 0; x < 16; ++x) f32_add2(tot[x], low[x], (g[0][x] + g[1][x]) + (g[2][x] + g[3][x]));
+  };
+  auto sync = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0);  // the chunk's loads, issued a chunk ago, and this wave's LDS reads
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  };
+  issue(st0, 0);
+  for (int i = 0; i < nch; i += 2) {
+    sync();
+    issue(st1, i + 1);
+    chunk(st0, i);
+    if (i + 1 < nch) {
+      sync();
+      issue(st0, i + 2);
+      chunk(st1, i + 1);
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0);  // no direct load outlives the workgroup's LDS
+  if constexpr (KW == 1) {
+#pragma unroll
+    for (int x = 0; x < 16; ++x) {
+      const int m = m0 + 32 * wm + 8 * (x >> 2) + 4 * hl + (x & 3), n = n0 + 32 * wn + r;
+      if (m < M && n < N) epi_apply<EPI>(e, m, n, f32_round2(tot[x], low[x]));
+    }
+  } else {
+    __syncthreads();  // the stages become the waves' partial tiles
+    typedef float Part[32][33];
+    Part *hi = (Part*)&st0[0], *lo = (Part*)&st1[0];
+    static_assert(sizeof(F32Stage) >= sizeof(Part), "a wave's partial tile");
+#pragma unroll
+    for (int x = 0; x < 16; ++x) {
+      hi[wave][8 * (x >> 2) + 4 * hl + (x & 3)][r] = tot[x];
+      lo[wave][8 * (x >> 2) + 4 * hl + (x & 3)][r] = low[x];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 16 / KW; ++u) {
+      const int rr = (threadIdx.x >> 5) + 2 * KW * u, cc = threadIdx.x & 31;
+      float v = hi[0][rr][cc], c = lo[0][rr][cc];
+#pragma unroll
+      for (int w = 1; w < KW; ++w) {
+        f32_add2(v, c, hi[w][rr][cc]);
+        c += lo[w][rr][cc];
+      }
+      if (m0 + rr < M && n0 + cc < N) epi_apply<EPI>(e, m0 + rr, n0 + cc, f32_round2(v, c));
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1590,6 +1747,26 @@ static void launch_gemv(const void* A, const void* W, int M, const int* Mdev, in
   else launch_gemv_mb<T, 8>(A, W, M, Mdev, N, K, e, s);
 }
 
+static void launch_f32(const void* A, const void* W, int Mcap, const int* Mdev, int Mtyp, int N, int K, const Epi& e,
+                       hipStream_t s) {
+  // 64 x 64 tiles once they give every CU two (a wave per SIMD each); eight
+  // waves where a CU has no more than one tile and each has two chunks at least
+  const bool wide = (int64_t)((Mtyp + 63) / 64) * ((N + 63) / 64) >= 512;
+  const bool few = (int64_t)((Mtyp + 31) / 32) * ((N + 31) / 32) <= 256 && K >= 512;
+  const int T = wide ? 64 : 32, ntiles = (N + T - 1) / T, mtiles = (Mcap + T - 1) / T;
+  const dim3 grid((unsigned)(ntiles * mtiles));
+  const float *a = (const float*)A, *w = (const float*)W;
+  if (wide)
+    FC_EPI_SWITCH(e.mode,
+                  hipLaunchKernelGGL((k_gemm_f32<1, E>), grid, dim3(256), 0, s, a, w, Mcap, Mdev, N, K, ntiles, e))
+  else if (few)
+    FC_EPI_SWITCH(e.mode,
+                  hipLaunchKernelGGL((k_gemm_f32<8, E>), grid, dim3(512), 0, s, a, w, Mcap, Mdev, N, K, ntiles, e))
+  else
+    FC_EPI_SWITCH(e.mode,
+                  hipLaunchKernelGGL((k_gemm_f32<4, E>), grid, dim3(256), 0, s, a, w, Mcap, Mdev, N, K, ntiles, e))
+}
+
 // register ring depth of the K-split kernel: 4 chunks for the 32 x 16 and
 // 32 x 32 tiles (the draft's weight streams: few columns per wave), else 3
 template <int MB, int NB, bool PK = false, int NS = (MB == 2 && NB <= 2) ? 4 : 3>
@@ -1955,7 +2132,14 @@ int fc_launch_gemm(const void* A, const void* W, int Mcap, const int* Mdev, int 
     *splits = p.S;
   }
   if (p.gemv) {
-    launch_gemv<float>(A, W, Mcap, Mdev, N, K, ee, s);
+    // Up to 16 rows k_gemv reads the weights twice at most (16 x 256 x 1024: 11.5 us
+    // against 12); where the 32 x 32 tiles leave three CUs in four without one
+    // and K is long, its column per wave spreads the work better (24 x 768 x 3072:
+    // 22.5 against 28). The tiles' 16-byte loads want their operands on that boundary.
+    const bool starved = (int64_t)((Mtyp + 31) / 32) * ((N + 31) / 32) <= 64 && K > 1024;
+    if (Mtyp <= GEMV_MAX_M || starved || (((uintptr_t)A | (uintptr_t)W) & 15) != 0)
+      launch_gemv<float>(A, W, Mcap, Mdev, N, K, ee, s);
+    else launch_f32(A, W, Mcap, Mdev, Mtyp, N, K, ee, s);
   } else if (p.big) {
     FC_CHECK_ARG(ee.rms_in == nullptr && ee.xa == nullptr, "the 256 x 256 GEMM has no folded-norm epilogue");
     launch_big(A, W, Mcap, Mdev, N, K, p.mb, p.nb, p.S, ee, s);
