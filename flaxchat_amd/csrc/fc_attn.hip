@@ -24,8 +24,9 @@
 // The four waves merge in LDS; splits merge in k_attn_combine.
 // Prefill-width chunks (>= 128 query columns per row) take k_attn_pf: 128
 // columns per workgroup on the 32x32x16 MFMA, K/V tiles shared through LDS.
-// fp32 path (parity mode, or head_dim != 128): one workgroup per query with
-// the reference's operation order (scores, max, exp, normalise, weighted sum).
+// fp32 path (parity mode): k_attn_f32 on the fp32 matrix cores. head_dim != 128:
+// k_attn_valu, one workgroup per query with the reference's operation order
+// (scores, max, exp, normalise, weighted sum).
 #include "fc_common.h"
 #include "fc_internal.h"
 #include <mutex>
@@ -856,7 +857,180 @@ __global__ __launch_bounds__(256) void k_attn_combine(const float* __restrict__ 
 }
 
 // ---------------------------------------------------------------------------
-// VALU attention, reference operation order (fp32 parity path, any hd <= 128)
+// fp32 attention on the fp32 matrix cores (head_dim 128, the parity mode): a
+// workgroup owns 32 query columns (token, head in group) of one (row, KV
+// group); its eight waves take every eighth 32-key tile, each with its own
+// online softmax, and are merged in LDS. Per tile and wave S^T = K Q^T and
+// O^T += V^T P^T are 64 32x32x2 MFMAs each; lane l holds column l % 32 and its
+// operands come 16 bytes at a time, 4 k of half l / 32 (the order of dims and
+// of keys is free), which makes the scores' registers the P operand as they
+// stand. k_attn_valu gives one query to a workgroup, whose threads each walk
+// whole key rows: 2 x 500 queries, 2 heads, window 256: 132 -> 27 us; one query
+// of 1000 keys 76 -> 50, of 10 18.6 -> 18.4. Bound by the latency of one wave's
+// tiles (its loads wait for each other: 256 VGPRs hold no second tile).
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ f32x16 mfma32fa(float a, float b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+#define AF_WAVES 8
+__global__ __launch_bounds__(64 * AF_WAVES, 2) void k_attn_f32(const float* __restrict__ q,
+                                                               const float* __restrict__ kc,
+                                                               const float* __restrict__ vc, float* __restrict__ y,
+                                                               int H, int G, int cap, const int* __restrict__ row_off,
+                                                               const int* __restrict__ start, int max_per_row,
+                                                               int Mcap, int window, float scale) {
+  constexpr int HD = 128;
+  const int bg = blockIdx.y, b = bg / G, g = bg - b * G, rep = H / G;
+  const RowSpan sp = row_span(row_off, b, max_per_row, Mcap);
+  const int base = sp.base, n = sp.n, s0 = start[b];
+  const int ncol = n * rep, c0 = blockIdx.x * 32;
+  if (c0 >= ncol) return;  // the whole workgroup
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, hl = lane >> 5;
+  const int col = c0 + (lane & 31);
+  const bool cvalid = col < ncol;
+  const int j = cvalid ? col / rep : 0, head = g * rep + (cvalid ? col - j * rep : 0);
+  // a position past the cache sees what its last position sees
+  const int pos_c = min(s0 + j, cap - 1), lo_c = window > 0 ? max(0, pos_c - window) : 0;
+  const int p_hi = min(s0 + min(c0 + 31, ncol - 1) / rep, cap - 1);
+  const int p_lo = min(s0 + c0 / rep, cap - 1);
+  const int t0 = (window > 0 ? max(0, p_lo - window) : 0) & ~31;
+  const int ntiles = (p_hi - t0 + 32) >> 5;
+  float4 qf[16];  // dims 8 j + 4 hl .. +3 of this lane's query
+  {
+    const float* qr = q + ((int64_t)(base + j) * H + head) * HD + 4 * hl;
+#pragma unroll
+    for (int d = 0; d < 16; ++d) qf[d] = *(const float4*)(qr + 8 * d);
+  }
+  const float* kb = kc + (int64_t)bg * cap * HD;
+  const float* vb = vc + (int64_t)bg * cap * HD;
+  __shared__ float xo[AF_WAVES / 2][64][64], xm[AF_WAVES / 2][2][64];
+  float m_run = -INFINITY, l_run = 0.f;
+  f32x16 O[4];  // dims 32 dd + 8 (x / 4) + 4 hl + x % 4 of this lane's column
+#pragma unroll
+  for (int dd = 0; dd < 4; ++dd)
+#pragma unroll
+    for (int x = 0; x < 16; ++x) O[dd][x] = 0.f;
+  for (int t = wave; t < ntiles; t += AF_WAVES) {
+    const int k0 = t0 + 32 * t;  // a multiple of 32 below cap
+    float4 kf[16];
+    const float* kr = kb + (int64_t)(k0 + (lane & 31)) * HD + 4 * hl;
+#pragma unroll
+    for (int d = 0; d < 16; ++d) kf[d] = *(const float4*)(kr + 8 * d);
+    f32x16 s2[2];
+#pragma unroll
+    for (int x = 0; x < 16; ++x) s2[0][x] = s2[1][x] = 0.f;
+#pragma unroll
+    for (int d = 0; d < 16; ++d) {
+      s2[d & 1] = mfma32fa(kf[d].x, qf[d].x, s2[d & 1]);
+      s2[d & 1] = mfma32fa(kf[d].y, qf[d].y, s2[d & 1]);
+      s2[d & 1] = mfma32fa(kf[d].z, qf[d].z, s2[d & 1]);
+      s2[d & 1] = mfma32fa(kf[d].w, qf[d].w, s2[d & 1]);
+    }
+    float p[16], mt = -INFINITY;
+#pragma unroll
+    for (int x = 0; x < 16; ++x) {
+      const int key = k0 + 8 * (x >> 2) + 4 * hl + (x & 3);
+      const bool ok = cvalid && key >= lo_c && key <= pos_c;
+      p[x] = ok ? (s2[0][x] + s2[1][x]) * scale : -INFINITY;
+      mt = fmaxf(mt, p[x]);
+    }
+    mt = fmaxf(mt, __shfl_xor(mt, 32, WAVE));
+    const float m_new = fmaxf(m_run, mt), m_use = m_new == -INFINITY ? 0.f : m_new;
+    if (__any(m_new > m_run)) {
+      const float alpha = expf(m_run - m_use);
+      l_run *= alpha;
+#pragma unroll
+      for (int dd = 0; dd < 4; ++dd) O[dd] *= alpha;
+      m_run = m_new;
+    }
+#pragma unroll
+    for (int x = 0; x < 16; ++x) {
+      p[x] = expf(p[x] - m_use);
+      l_run += p[x];
+    }
+    // V blocks of 32 keys are [128 dims][32]: keys 8 jj + 4 hl .. +3 of dim 32 dd + l % 32
+    const float* vt = vb + (int64_t)k0 * HD;
+    // a key that some column does not see counts as 0 there even where its V
+    // is not finite (slots past the row's end hold anything): key by key then
+    bool odd = false;
+    if (k0 + 31 > p_lo || (window > 0 && k0 < p_hi - window)) {
+#pragma unroll 4
+      for (int i = 0; i < 16; ++i) {
+        const float4 f = *(const float4*)(vt + 256 * i + 4 * lane);
+        const float z = (f.x * 0.f + f.y * 0.f) + (f.z * 0.f + f.w * 0.f);  // NaN unless all are finite
+        odd |= z != z;
+      }
+    }
+    if (__any(odd)) {
+      float(*pw)[32] = (float(*)[32])((float*)xo + wave * 1024);  // this wave's P, [key][column]
+#pragma unroll
+      for (int x = 0; x < 16; ++x) pw[8 * (x >> 2) + 4 * hl + (x & 3)][lane & 31] = p[x];
+      __builtin_amdgcn_wave_barrier();
+      for (int kk = 0; kk < 32; ++kk) {
+        const bool sees = k0 + kk >= lo_c && k0 + kk <= pos_c;
+        const float pk = pw[kk][lane & 31];
+#pragma unroll
+        for (int dd = 0; dd < 4; ++dd)
+#pragma unroll
+          for (int x = 0; x < 16; ++x) {
+            const float v = vt[(32 * dd + 8 * (x >> 2) + 4 * hl + (x & 3)) * 32 + kk];
+            O[dd][x] = sees ? fmaf(pk, v, O[dd][x]) : O[dd][x];
+          }
+      }
+      __builtin_amdgcn_wave_barrier();
+      continue;
+    }
+#pragma unroll
+    for (int dd = 0; dd < 4; ++dd) {
+      float4 vf[4];
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) vf[jj] = *(const float4*)(vt + dd * 1024 + (lane & 31) * 32 + 8 * jj + 4 * hl);
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {
+        O[dd] = mfma32fa(vf[jj].x, p[4 * jj], O[dd]);
+        O[dd] = mfma32fa(vf[jj].y, p[4 * jj + 1], O[dd]);
+        O[dd] = mfma32fa(vf[jj].z, p[4 * jj + 2], O[dd]);
+        O[dd] = mfma32fa(vf[jj].w, p[4 * jj + 3], O[dd]);
+      }
+    }
+  }
+  // merge the waves, half of the rest giving its O, maximum and sum to the other half each time
+  l_run += __shfl_xor(l_run, 32, WAVE);
+#pragma unroll
+  for (int half = AF_WAVES / 2; half >= 1; half >>= 1) {
+    __syncthreads();
+    if (wave >= half && wave < 2 * half) {
+#pragma unroll
+      for (int dd = 0; dd < 4; ++dd)
+#pragma unroll
+        for (int x = 0; x < 16; ++x) xo[wave - half][16 * dd + x][lane] = O[dd][x];
+      xm[wave - half][0][lane] = m_run;
+      xm[wave - half][1][lane] = l_run;
+    }
+    __syncthreads();
+    if (wave < half) {
+      const float m1 = xm[wave][0][lane], m = fmaxf(m_run, m1), mu = m == -INFINITY ? 0.f : m;
+      const float a0 = expf(m_run - mu), a1 = expf(m1 - mu);
+      l_run = l_run * a0 + xm[wave][1][lane] * a1;
+#pragma unroll
+      for (int dd = 0; dd < 4; ++dd)
+#pragma unroll
+        for (int x = 0; x < 16; ++x) O[dd][x] = O[dd][x] * a0 + xo[wave][16 * dd + x][lane] * a1;
+      m_run = m;
+    }
+  }
+  if (wave != 0 || !cvalid) return;
+  float* yr = y + (int64_t)(base + j) * H * HD + head * HD + 4 * hl;
+#pragma unroll
+  for (int dd = 0; dd < 4; ++dd)
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      *(float4*)(yr + 32 * dd + 8 * u) = make_float4(O[dd][4 * u] / l_run, O[dd][4 * u + 1] / l_run,
+                                                     O[dd][4 * u + 2] / l_run, O[dd][4 * u + 3] / l_run);
+}
+
+// ---------------------------------------------------------------------------
+// VALU attention, reference operation order (any hd <= 128)
 // ---------------------------------------------------------------------------
 #define VALU_MAXK 8192
 template <typename T>
@@ -1014,7 +1188,13 @@ int fc_launch_attention(const void* q, const void* kc, const void* vc, void* y, 
     FC_CHECK_ARG(hd <= 128, "head_dim must be <= 128");
     FC_CHECK_ARG(max_keys <= VALU_MAXK, "VALU attention supports at most 8192 visible keys");
     const dim3 grid(max_per_row, H, B);
-    if (dtype == FC_BF16)
+    // 16-byte operand loads: every array on its boundary (head_dim 128 keeps the rows on it)
+    const bool vec = (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc | (uintptr_t)y) & 15) == 0;
+    if (dtype == FC_F32 && hd == 128 && vec && (int64_t)B * G <= 65535)
+      hipLaunchKernelGGL(k_attn_f32, dim3((max_per_row * (H / G) + 31) / 32, B * G), dim3(64 * AF_WAVES), 0, s,
+                         (const float*)q, (const float*)kc, (const float*)vc, (float*)y, H, G, cap, row_off, start,
+                         max_per_row, max_tokens, window, scale);
+    else if (dtype == FC_BF16)
       hipLaunchKernelGGL(k_attn_valu<bf16_t>, grid, dim3(256), 0, s, (const bf16_t*)q, (const bf16_t*)kc,
                          (const bf16_t*)vc, (bf16_t*)y, H, G, hd, cap, row_off, start, max_per_row, max_tokens,
                          window, scale, rows);

@@ -1,9 +1,13 @@
 """The fp32 matrix-core kernels: k_gemm_f32's two tilings at ragged rows,
-columns and K tails, every epilogue of fc_gemm, against float64. The error must
-not exceed what sequential fp32 sums would show."""
+columns and K tails, every epilogue of fc_gemm, against float64; and fp32
+attention over ragged rows, GQA, windows and key counts around its 32-key
+tiles. Their error must not exceed what sequential fp32 sums would show."""
+
+import numpy as np
 import pytest
 
 torch = pytest.importorskip("torch")
+import flaxchat_amd.torch_ops  # noqa: E402,F401
 from flaxchat_amd._lib import check, lib  # noqa: E402
 
 pytestmark = pytest.mark.gpu
@@ -32,6 +36,38 @@ def test_fp32_gemm(M, N, K, epi):
     assert err <= 4 * 2.0 ** -24, err
 
 
+@pytest.mark.parametrize("H,G,n,start,window", [
+    (2, 2, [1, 1, 1], [0, 31, 500], 0), (2, 2, [33, 0, 7], [0, 0, 300], 100), (6, 2, [5, 64], [63, 10], 0),
+    (12, 4, [1, 9], [1000, 0], 0), (2, 2, [500, 499], [0, 0], 256), (4, 1, [3], [40], 8)])
+def test_fp32_attention(H, G, n, start, window):
+    print(f"H={H} G={G} n={n} start={start} window={window}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(len(n) + H)
+    B, cap = len(n), (max(a + b for a, b in zip(n, start)) + 31) // 32 * 32
+    off = np.concatenate([[0], np.cumsum(n)]).astype(np.int32)
+    q = torch.randn(int(off[-1]), H, 128, device="cuda", generator=g) * 2
+    k = torch.randn(B, G, cap, 128, device="cuda", generator=g)
+    v = torch.randn(B, G, cap, 128, device="cuda", generator=g)
+    vb = v.view(B, G, cap // 32, 32, 128).transpose(3, 4).contiguous()
+    got = torch.ops.flaxchat_mi355x.attention(q, k, vb, torch.from_numpy(off).cuda(),
+                                              torch.tensor(start, dtype=torch.int32, device="cuda"), max(n), window)
+    rep = H // G
+    for b in range(B):
+        if n[b] == 0:
+            continue
+        end = start[b] + n[b]
+        qb = q[off[b]:off[b + 1]].double().transpose(0, 1)
+        kb, vv = (t[b, :, :end].double().repeat_interleave(rep, 0) for t in (k, v))
+        pos = torch.arange(start[b], end, device="cuda")[:, None]
+        key = torch.arange(end, device="cuda")[None]
+        see = (key <= pos) & ((pos - key <= window) if window > 0 else True)
+        s = (torch.matmul(qb, kb.transpose(1, 2).contiguous()) / np.sqrt(128)).masked_fill(~see, -np.inf)
+        want = torch.matmul(torch.softmax(s, -1), vv).transpose(0, 1).reshape(n[b], -1)
+        # scores of up to ~12 from 128 products (two chains of 64 / 2): ~8 roundings, through exp
+        # as a relative error; at most 64 rescalings and 32-key sums
+        err = float((got[off[b]:off[b + 1]] - want).abs().max())
+        assert err <= 100 * 2.0 ** -24 * 4, err
+
+
 @pytest.mark.parametrize("M,N,K", [(33, 100, 24), (1000, 8192, 256)])
 def test_fp32_gemm_infinities(M, N, K):
     """An overflowing or infinite sum is infinite, as a plain sum is; other outputs are untouched."""
@@ -50,3 +86,30 @@ def test_fp32_gemm_infinities(M, N, K):
     want[1], want[2], want[3] = float("inf"), float("nan"), float("inf")
     want[1, N - 1] = -float("inf")
     assert bool(torch.equal(torch.nan_to_num(out, 1e4, 2e4, -2e4), torch.nan_to_num(want, 1e4, 2e4, -2e4)))
+
+
+def test_fp32_attention_unseen_keys():
+    """Keys a query does not see, past the row's end, after it or left of its window, do not
+    reach it even where their K and V are infinite or NaN; the queries that see one do get it."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    n, start, window, cap = 40, 50, 20, 128
+    q = torch.randn(n, 2, 128, device="cuda", generator=g)
+    k = torch.randn(1, 2, cap, 128, device="cuda", generator=g)
+    v = torch.randn(1, 2, cap, 128, device="cuda", generator=g)
+    off, st = torch.tensor([0, n], dtype=torch.int32).cuda(), torch.tensor([start], dtype=torch.int32).cuda()
+
+    def run():
+        vb = v.view(1, 2, cap // 32, 32, 128).transpose(3, 4).contiguous()
+        return torch.ops.flaxchat_mi355x.attention(q, k, vb, off, st, n, window)
+
+    clean = run().clone()
+    k[:, :, start + n:], v[:, :, start + n:] = float("nan"), float("nan")
+    k[:, :, :start - window], v[:, :, :start - window] = float("nan"), float("inf")
+    v[:, 1, start + 20] = float("inf")  # seen by queries 20 .. 39 of head 1 (window 20: up to 40)
+    got = run()
+    seen = torch.zeros(n, 2, 128, dtype=torch.bool, device="cuda")
+    seen[20:, 1] = True
+    seen = seen.view(n, -1)
+    assert bool(torch.isinf(got[seen]).all())
+    # the same terms by FMA instead of by the matrix cores: a few roundings
+    assert float((got - clean)[~seen].abs().max()) <= 64 * 2.0 ** -24
