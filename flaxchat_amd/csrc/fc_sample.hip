@@ -255,23 +255,28 @@ __device__ __forceinline__ float row_sum(float v, RegSmem& sm) {
   return v;
 }
 
+// The row into registers by 16-byte loads wherever it starts (global loads need
+// only their entries' own 4-byte boundary), its last V % 4 entries one by one.
+// A row off the 16-byte boundary entry by entry, as before, is four loads per
+// line instead of one: 128 rows x 39330, T = 0: 22.9 -> 16.8 us.
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 template <int NQ>
-__device__ __forceinline__ void reg_load_row(const float* __restrict__ z, int V, bool vec, float (&v)[NQ][4]) {
-  if (vec) {  // 16-byte aligned row, V % 4 == 0: whole groups
+__device__ __forceinline__ void reg_load_row(const float* __restrict__ z, int V, float (&v)[NQ][4]) {
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      const int e = 4 * (NTHR * q + (int)threadIdx.x);
-      float4 t = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-      if (e < V) t = *(const float4*)(z + e);
-      v[q][0] = t.x; v[q][1] = t.y; v[q][2] = t.z; v[q][3] = t.w;
-    }
-  } else {
+  for (int q = 0; q < NQ; ++q) {
+    const int e = 4 * (NTHR * q + (int)threadIdx.x);
+    f32x4_a4 t = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    if (e + 4 <= V) t = *(const f32x4_a4*)(z + e);
+    v[q][0] = t.x; v[q][1] = t.y; v[q][2] = t.z; v[q][3] = t.w;
+  }
+  const int g = V >> 2;  // the group past the last whole one
+  if ((V & 3) != 0 && (int)threadIdx.x == g % NTHR) {
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      const int e = 4 * (NTHR * q + (int)threadIdx.x);
+    for (int q = 0; q < NQ; ++q)
+      if (q == g / NTHR)
 #pragma unroll
-      for (int w = 0; w < 4; ++w) v[q][w] = e + w < V ? z[e + w] : -INFINITY;
-    }
+        for (int w = 0; w < 3; ++w)
+          if (4 * g + w < V) v[q][w] = z[4 * g + w];
   }
 }
 
@@ -434,13 +439,13 @@ __device__ __forceinline__ void put_stat(const StatOut& o, int row, const fc_row
 // NQ = 0: rows longer than 65536 entries (read from memory in every step).
 template <int NQ>
 __global__ __launch_bounds__(NTHR) void k_row_stats(const float* __restrict__ logits, int V, float T, int top_k,
-                                                    int vec, StatOut out) {
+                                                    StatOut out) {
   const float* z = logits + (int64_t)blockIdx.x * V;
   if constexpr (NQ > 0) {
     __shared__ RegSmem rs;
     float v[NQ][4];
     fc_rowstat r;
-    reg_load_row<NQ>(z, V, vec != 0, v);
+    reg_load_row<NQ>(z, V, v);
     if (reg_row_stats<NQ>(v, V, T, top_k, r, rs)) {
       if (threadIdx.x == 0) put_stat(out, blockIdx.x, r);
       return;
@@ -453,12 +458,10 @@ __global__ __launch_bounds__(NTHR) void k_row_stats(const float* __restrict__ lo
 
 // groups of four entries per thread that hold a row of V entries (0: too long)
 static int reg_nq(int V) { return V <= 4 * NTHR * 4 ? 4 : V <= 4 * NTHR * 8 ? 8 : V <= 4 * NTHR * 16 ? 16 : 0; }
-static int rows_vec(const float* z, int V) { return V % 4 == 0 && (uintptr_t)z % 16 == 0; }
 
 static int launch_row_stats(const float* logits, int rows, int V, float T, int top_k, const StatOut& o, hipStream_t s) {
   if (rows <= 0) return FC_OK;
-  const int vec = rows_vec(logits, V);
-#define ROW_STATS(NQ) hipLaunchKernelGGL(k_row_stats<NQ>, dim3(rows), dim3(NTHR), 0, s, logits, V, T, top_k, vec, o)
+#define ROW_STATS(NQ) hipLaunchKernelGGL(k_row_stats<NQ>, dim3(rows), dim3(NTHR), 0, s, logits, V, T, top_k, o)
   switch (reg_nq(V)) {
     case 4: ROW_STATS(4); break;
     case 8: ROW_STATS(8); break;
@@ -1671,7 +1674,7 @@ extern "C" int32_t fc_spec_round(const fc_model* target, const fc_cache* tcache,
 // NQ: the row in registers (reg_row_stats), 0 for rows longer than 65536.
 template <bool ENGINE, int NQ>
 __global__ __launch_bounds__(NTHR) void k_fast_sample(const float* __restrict__ logits, int V, float T, int top_k,
-                                                      int vec, uint64_t seed, int eos, int* __restrict__ gen,
+                                                      uint64_t seed, int eos, int* __restrict__ gen,
                                                       int gen_cap, int* __restrict__ pos, int* __restrict__ done,
                                                       int* __restrict__ step, const int* __restrict__ max_pos,
                                                       const int* __restrict__ forced, int* __restrict__ tok_cur,
@@ -1699,7 +1702,7 @@ __global__ __launch_bounds__(NTHR) void k_fast_sample(const float* __restrict__ 
     if constexpr (NQ > 0) {
       __shared__ RegSmem rsm;
       float v[NQ][4];
-      reg_load_row<NQ>(z, V, vec != 0, v);
+      reg_load_row<NQ>(z, V, v);
       reg = reg_row_stats<NQ>(v, V, T, top_k, rs, rsm);
       if (reg && tid == 0) stats[b] = rs;
       if (reg && T > 0.f) {
@@ -1762,9 +1765,8 @@ template <bool ENGINE>
 static int launch_fast_sample(const float* logits, int batch, int V, float T, int top_k, uint64_t seed, int eos,
                               int* gen, int gen_cap, int* pos, int* done, int* step, const int* max_pos,
                               const int* forced, int* tok_cur, fc_rowstat* stats, hipStream_t s) {
-  const int vec = rows_vec(logits, V);
 #define FAST_SAMPLE(NQ)                                                                                         \
-  hipLaunchKernelGGL((k_fast_sample<ENGINE, NQ>), dim3(batch), dim3(NTHR), 0, s, logits, V, T, top_k, vec, seed, \
+  hipLaunchKernelGGL((k_fast_sample<ENGINE, NQ>), dim3(batch), dim3(NTHR), 0, s, logits, V, T, top_k, seed, \
                      eos, gen, gen_cap, pos, done, step, max_pos, forced, tok_cur, stats)
   switch (reg_nq(V)) {
     case 4: FAST_SAMPLE(4); break;

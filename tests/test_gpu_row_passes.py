@@ -42,7 +42,7 @@ def _upload(z, off):
     return t
 
 
-@pytest.mark.parametrize("V", [1, 3, 1000, 4099, 16384, 16385, 32768, 65535, 65536, 65540])
+@pytest.mark.parametrize("V", [1, 3, 1000, 4098, 4099, 16384, 16385, 32768, 65535, 65536, 65540])
 @pytest.mark.parametrize("top_k,T", [(40, 0.8), (1, 1.0), (130, 0.8), (1024, 1.0), (1500, 0.7), (0, 0.8), (40, 0.0)])
 def test_row_stats_and_sample(V, top_k, T):
     from oracle.sampling import fast_sample, topk_keep
