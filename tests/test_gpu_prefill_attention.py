@@ -1,7 +1,7 @@
 """Prefill-width attention: the one- and two-group kernels at ragged rows
 (empty and one-token rows among them), GQA groups whose columns straddle
 tokens, windows, key counts around its 64-key steps, and row-major against
-operand-order output."""
+operand-order output. And the merge of the decode kernels' key splits."""
 
 import numpy as np
 import pytest
@@ -33,6 +33,16 @@ def _reference(q, k, v, n, start, off, window):
     return out
 
 
+def _layouts(k, v):
+    """The caches' layouts: K blocks of 32 keys in K.Q^T fragment order, V blocks transposed."""
+    B, G, cap = k.shape[:3]
+    kb = torch.empty_like(k)
+    kk, d = torch.arange(32, device="cuda")[:, None], torch.arange(128, device="cuda")[None]
+    e = ((2 * (d // 32) + (kk // 4) % 2) * 64 + 4 * (kk // 8) + kk % 4 + 16 * ((d // 8) % 4)) * 8 + d % 8
+    kb.view(B, G, cap // 32, 4096)[..., e.reshape(-1)] = k.view(B, G, cap // 32, 4096)
+    return kb, v.view(B, G, cap // 32, 32, 128).transpose(3, 4).contiguous()
+
+
 # (heads, groups, tokens per row, first positions, window): up to 256 workgroups
 # take two groups of waves, more one
 CASES = [(2, 2, [128], [0], 0), (2, 2, [129, 0, 1, 200], [0, 0, 700, 63], 0), (12, 4, [43, 100, 7], [500, 0, 64], 100),
@@ -52,12 +62,7 @@ def test_prefill_attention(H, G, n, start, window):
     q = (torch.randn(tot, H, 128, device="cuda", generator=gen) * 2).to(torch.bfloat16)
     k = (torch.randn(B, G, cap, 128, device="cuda", generator=gen) * 1.5).to(torch.bfloat16)
     v = torch.randn(B, G, cap, 128, device="cuda", generator=gen).to(torch.bfloat16)
-    # the caches' layouts: K blocks of 32 keys in K.Q^T fragment order, V blocks transposed
-    kb = torch.empty_like(k)
-    kk, d = torch.arange(32, device="cuda")[:, None], torch.arange(128, device="cuda")[None]
-    e = ((2 * (d // 32) + (kk // 4) % 2) * 64 + 4 * (kk // 8) + kk % 4 + 16 * ((d // 8) % 4)) * 8 + d % 8
-    kb.view(B, G, cap // 32, 4096)[..., e.reshape(-1)] = k.view(B, G, cap // 32, 4096)
-    vb = v.view(B, G, cap // 32, 32, 128).transpose(3, 4).contiguous()
+    kb, vb = _layouts(k, v)
     ro, st = torch.from_numpy(off).cuda(), torch.tensor(start, dtype=torch.int32, device="cuda")
     mpr = max(max(n), -(-128 * G // H))  # prefill width: at least 128 columns per row and group
     got = torch.ops.flaxchat_mi355x.attention(q, kb, vb, ro, st, mpr, window)
@@ -73,3 +78,25 @@ def test_prefill_attention(H, G, n, start, window):
                              ro.data_ptr(), st.data_ptr(), window, max_keys, _lib.FC_BF16, ws.data_ptr(), ws.numel(),
                              torch.cuda.current_stream().cuda_stream), "fc_attention")
     assert torch.equal(tops.frag_to_rows(y, tot), got)
+
+
+# key splits of 128 keys: 1, 2, 8, 9, 16, 17 and 43; splits past a short row's end and before a
+# window hold nothing; empty rows; 21 columns of a GQA group
+@pytest.mark.parametrize("H,G,n,start,window", [
+    (6, 6, [1], [100], 0), (6, 6, [1], [254], 0), (6, 6, [1], [1022], 0), (6, 6, [1], [1024], 0),
+    (6, 6, [1], [2047], 0), (6, 6, [1], [2048], 0), (6, 6, [1, 0, 1], [2048, 5, 10], 0), (6, 6, [1], [5600], 0),
+    (12, 4, [7, 3], [5400, 900], 0), (6, 6, [5], [3000], 1024)])
+def test_key_split_merge(H, G, n, start, window):
+    print(f"H={H} G={G} n={n} start={start} window={window}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(start[0] + H)
+    B, cap = len(n), (max(a + b for a, b in zip(n, start)) + 31) // 32 * 32
+    off = np.concatenate([[0], np.cumsum(n)]).astype(np.int32)
+    q = (torch.randn(int(off[-1]), H, 128, device="cuda", generator=gen) * 2).to(torch.bfloat16)
+    k = (torch.randn(B, G, cap, 128, device="cuda", generator=gen) * 1.5).to(torch.bfloat16)
+    v = torch.randn(B, G, cap, 128, device="cuda", generator=gen).to(torch.bfloat16)
+    kb, vb = _layouts(k, v)
+    ro, st = torch.from_numpy(off).cuda(), torch.tensor(start, dtype=torch.int32, device="cuda")
+    got = torch.ops.flaxchat_mi355x.attention(q, kb, vb, ro, st, max(n), window)
+    want = _reference(q, k, v, n, start, off, window)
+    # P and the output are rounded to bf16 (2^-9 relative each), P against values below ~4.5
+    assert float((got.double() - want).abs().max()) <= 2 * 2.0 ** -9 * 4.5 + 2.0 ** -9
