@@ -1917,6 +1917,13 @@ static bool big_rows(int M, int N) {
   return N % 128 == 0 && (int64_t)((M + 63) / 64) * (N / 64) > 512;
 }
 
+// A residual GEMM with a deep K (the MLP c_proj) that may split it is the
+// faster there from FC_MID_M rows on: with the split its tiles fill the CUs,
+// while a 64 x 64 tile of k_gemm_dma walks all of K alone.
+// Whole chunks, us, without and with: 4 layers of 1536 at 900 rows 880 / 812, at
+// 1152 rows (4 KV heads) 1064 / 1007; of 768 at 1080 rows (12 layers) 611 / 548.
+static bool big_deep(int M, int N, int K) { return M >= FC_MID_M && N % 128 == 0 && K >= 2048; }
+
 // The cheapest tile and K split (S of at most s_max, each split's partials
 // written and read back once by the RMSNorm that sums them, at ~4 TB/s). A
 // split needs at least 8 k steps.
@@ -1955,7 +1962,7 @@ static GemmPlan plan_gemm(int Mtyp, int N, int K, int dtype, bool can_split) {
       return p;
     }
   }
-  if (big_rows(Mtyp, N)) {
+  if (big_rows(Mtyp, N) || (can_split && big_deep(Mtyp, N, K))) {
     p.big = true;
     big_tile(Mtyp, N, K, can_split ? FC_MAX_SPLIT : 1, p.mb, p.nb, p.S);
     return p;

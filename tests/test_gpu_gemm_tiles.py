@@ -92,3 +92,35 @@ def test_qkv_tile_matches_the_separate_prologue(M, D, kv):
                                    atol=2.0 ** -9)
     for a, b in ((got.k, want.k), (got.v, want.v)):
         np.testing.assert_allclose(a.float().cpu().numpy(), b.float().cpu().numpy(), rtol=2.0 ** -7, atol=2.0 ** -9)
+
+
+# rows past 832 with an n_embd whose MLP c_proj (K 3072, 6144) splits K on the large tiles
+@pytest.mark.parametrize("B,q,D,kv", [(93, 9, 768, 6), (119, 7, 768, 6), (128, 9, 1536, 4)])
+def test_split_residual_gemm_in_a_chunk(B, q, D, kv):
+    """A chunk against its rows in batches below those row counts (other GEMM
+    kernels): the same logits up to bf16 operand rounding."""
+    import flaxchat_amd.torch_ops  # noqa: F401
+    from flaxchat_amd.config import GPTConfig
+    from flaxchat_amd.runtime import DeviceCache, DeviceModel
+    print(f"B={B} q={q} D={D}", flush=True)
+    cfg = GPTConfig(sequence_len=512, vocab_size=1000, n_layer=2, n_head=D // 128, n_kv_head=kv, n_embd=D)
+    dm = DeviceModel.random_init(cfg, seed=2, dtype="bf16")
+    rng = np.random.default_rng(B)
+    tok = rng.integers(0, 1000, (B, q)).astype(np.int32)
+
+    def forward(t):
+        n = len(t)
+        cache = DeviceCache(dm, n, 64)
+        off = torch.arange(0, n * q + 1, q, dtype=torch.int32, device="cuda")
+        logits = torch.zeros(n, q, dm.V, device="cuda")
+        nb = lib().fc_forward_workspace_bytes(ctypes.byref(dm.desc), n, n * q, q, 0)
+        ws = torch.zeros(nb, device="cuda", dtype=torch.uint8)
+        torch.ops.flaxchat_mi355x.forward(ctypes.addressof(dm.desc), cache.k, cache.v, cache.hist,
+                                          torch.from_numpy(t.reshape(-1).copy()).cuda(), off,
+                                          torch.zeros(n, dtype=torch.int32, device="cuda"), q, q, logits, ws)
+        return logits.double()
+
+    got = forward(tok)
+    want = torch.cat([forward(tok[i:i + 32]) for i in range(0, B, 32)])
+    # bf16 operands (2^-9 each) through 2 layers: each side is within about 0.3% of float64
+    assert float((got - want).norm() / want.norm()) <= 0.012
