@@ -1921,7 +1921,7 @@ static bool big_rows(int M, int N) {
 // faster there from FC_MID_M rows on: with the split its tiles fill the CUs,
 // while a 64 x 64 tile of k_gemm_dma walks all of K alone.
 // Whole chunks, us, without and with: 4 layers of 1536 at 900 rows 880 / 812, at
-// 1152 rows (4 KV heads) 1064 / 1007; of 768 at 1080 rows (12 layers) 611 / 548.
+// 1152 rows (4 KV heads) 1064 / 1007; of 768 at 1080 rows 611 / 548.
 static bool big_deep(int M, int N, int K) { return M >= FC_MID_M && N % 128 == 0 && K >= 2048; }
 
 // The cheapest tile and K split (S of at most s_max, each split's partials
