@@ -601,22 +601,22 @@ __global__ __launch_bounds__(256 * KS, 2) void k_attn_pf(const bf16_t* __restric
   const int kend = min(s0 + lcol / rep + 1, cap);
   const int t0 = kbeg & ~31;
   const int ntiles = (kend - t0 + 31) >> 5, nstep = (ntiles + 1) >> 1;  // group grp takes steps grp, grp + KS, ..
-  // this wave's columns and key range
+  // this wave's columns and key range; positions past the cache end with the
+  // range (kend), behind which a step holds the last tile once more
   const int wc0 = c0 + 32 * wave;
   const bool wact = wc0 < ncol;
-  const int w_hi = wact ? s0 + min(wc0 + 31, ncol - 1) / rep : -1;
+  const int w_hi = wact ? min(s0 + min(wc0 + 31, ncol - 1) / rep, kend - 1) : -1;
   const int w_lo = window > 0 ? max(0, s0 + wc0 / rep - window) : 0;
   // keys inside [w_full_lo, w_full_hi] are visible to every column of the wave (no masks)
   const bool wfull = wc0 + 31 < ncol;
-  const int w_full_hi = s0 + wc0 / rep;  // the first column's position
+  const int w_full_hi = min(s0 + wc0 / rep, kend - 1);  // the first column's position
   const int w_full_lo = window > 0 ? max(0, s0 + (wc0 + 31) / rep - window) : 0;
   // this lane's column (query)
   const int col = wc0 + kk;
   const bool cvalid = col < ncol;
   const int j = cvalid ? col / rep : 0;
   const int head = g * rep + (cvalid ? col - (col / rep) * rep : 0);
-  const int pos_c = s0 + j;
-  const int lo_c = window > 0 ? max(0, pos_c - window) : 0;
+  const int hi_c = min(s0 + j, kend - 1), lo_c = window > 0 ? max(0, s0 + j - window) : 0;
   v4u qf[8];  // dims 16 h + 8 hl .. +7 of this lane's query
   {
     const bf16_t* qr = q + ((int64_t)(base + j) * H + head) * HD + 8 * hl;
@@ -695,7 +695,7 @@ __global__ __launch_bounds__(256 * KS, 2) void k_attn_pf(const bf16_t* __restric
 #pragma unroll
         for (int x = 0; x < 16; ++x) {
           const int kx = kb + 32 * u + 16 * (x >> 3) + 8 * hl + (x & 7);
-          if (!(cvalid && kx >= lo_c && kx <= pos_c)) sc[u][x] = -INFINITY;
+          if (!(cvalid && kx >= lo_c && kx <= hi_c)) sc[u][x] = -INFINITY;
         }
     }
     float m4[4];  // four chains each: one or two waves per SIMD leave latencies in sight

@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
 
 
 def _reference(q, k, v, n, start, off, window):
-    """float64 attention of packed rows over plain [B][G][cap][128] keys / values."""
+    """float64 attention of packed rows over plain [B][G][cap][128] keys / values; a query past
+    the cache's end sees what its window leaves of the cache, and one that sees no key gives 0."""
     out = torch.zeros(q.shape[0], q.shape[1] * 128, dtype=torch.float64, device=q.device)
     rep = q.shape[1] // k.shape[1]
     for b in range(len(n)):
@@ -26,10 +27,11 @@ def _reference(q, k, v, n, start, off, window):
         kb = k[b, :, :end].double().repeat_interleave(rep, 0)
         vb = v[b, :, :end].double().repeat_interleave(rep, 0)
         pos = torch.arange(start[b], end, device=q.device)[:, None]
-        key = torch.arange(end, device=q.device)[None]
+        key = torch.arange(kb.shape[1], device=q.device)[None]
         see = (key <= pos) & ((pos - key <= window) if window > 0 else True)
         s = (torch.matmul(qb, kb.transpose(1, 2).contiguous()) / np.sqrt(128)).masked_fill(~see, -np.inf)
-        out[off[b]:off[b + 1]] = torch.matmul(torch.softmax(s, -1), vb).transpose(0, 1).reshape(n[b], -1)
+        p = torch.softmax(s, -1).masked_fill(~see, 0.0)
+        out[off[b]:off[b + 1]] = torch.matmul(p, vb).transpose(0, 1).reshape(n[b], -1)
     return out
 
 
@@ -78,6 +80,30 @@ def test_prefill_attention(H, G, n, start, window):
                              ro.data_ptr(), st.data_ptr(), window, max_keys, _lib.FC_BF16, ws.data_ptr(), ws.numel(),
                              torch.cuda.current_stream().cuda_stream), "fc_attention")
     assert torch.equal(tops.frag_to_rows(y, tot), got)
+
+
+# rows that run past the cache's end: an odd number of 32-key tiles (3, 9, 5) and of 64-key
+# steps (5, 3), one and two groups of waves (two: 256 keys or more and few workgroups), a
+# first position behind the end, queries whose window lies behind it, GQA
+@pytest.mark.parametrize("H,G,n,start,window,cap", [
+    (2, 2, [130], [0], 0, 96), (2, 2, [300, 130], [0, 200], 0, 288), (2, 2, [400], [100], 100, 288),
+    (6, 2, [200, 64], [150, 288], 0, 288), (2, 2, [128], [300], 20, 288), (12, 4, [180] * 17, list(range(0, 340, 20)), 0,
+                                                                          160)])
+def test_prefill_attention_past_the_cache(H, G, n, start, window, cap):
+    """Every cached key counts once for a query at a position past the cache."""
+    print(f"H={H} G={G} n={n} start={start} window={window} cap={cap}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(len(n) + H)
+    B = len(n)
+    off = np.concatenate([[0], np.cumsum(n)]).astype(np.int32)
+    q = torch.randn(int(off[-1]), H, 128, device="cuda", generator=gen).to(torch.bfloat16)
+    k = torch.randn(B, G, cap, 128, device="cuda", generator=gen).to(torch.bfloat16)
+    v = torch.randn(B, G, cap, 128, device="cuda", generator=gen).to(torch.bfloat16)
+    kb, vb = _layouts(k, v)
+    ro, st = torch.from_numpy(off).cuda(), torch.tensor(start, dtype=torch.int32, device="cuda")
+    got = torch.ops.flaxchat_mi355x.attention(q, kb, vb, ro, st, max(n), window)
+    want = _reference(q, k, v, n, start, off, window)
+    # P and the output are rounded to bf16 (2^-9 relative each), P against values below ~4.5
+    assert float((got.double() - want).abs().max()) <= 2 * 2.0 ** -9 * 4.5 + 2.0 ** -9
 
 
 # key splits of 128 keys: 1, 2, 8, 9, 16, 17 and 43; splits past a short row's end and before a
