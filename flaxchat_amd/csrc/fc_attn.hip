@@ -697,6 +697,13 @@ __global__ __launch_bounds__(256 * KS, 2) void k_attn_pf(const bf16_t* __restric
           const int kx = kb + 32 * u + 16 * (x >> 3) + 8 * hl + (x & 7);
           if (!(cvalid && kx >= lo_c && kx <= hi_c)) sc[u][x] = -INFINITY;
         }
+      // a tile that no column of the wave sees: P is 0 there, and so has V to be, whose slots hold anything
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        if (kb + 32 * u > w_hi || kb + 32 * u + 31 < w_lo) {
+#pragma unroll
+          for (int f = 0; f < 8; ++f) vf[u][f] = v4u{0u, 0u, 0u, 0u};
+        }
     }
     float m4[4];  // four chains each: one or two waves per SIMD leave latencies in sight
 #pragma unroll

@@ -126,3 +126,30 @@ def test_key_split_merge(H, G, n, start, window):
     want = _reference(q, k, v, n, start, off, window)
     # P and the output are rounded to bf16 (2^-9 relative each), P against values below ~4.5
     assert float((got.double() - want).abs().max()) <= 2 * 2.0 ** -9 * 4.5 + 2.0 ** -9
+
+
+# NaN in the V of keys 96-127 reaches no query before them, of keys 64-95 no wave (32 queries)
+# whose windows start at key 96 or behind, though they lie in one 64-key step with keys it sees
+@pytest.mark.parametrize("bad,window,clean", [(range(96, 128), 0, range(0, 96)),
+                                              (range(64, 96), 40, [*range(0, 64), *range(160, 300)])])
+@pytest.mark.parametrize("cap", [320, 1024])
+@pytest.mark.parametrize("B", [1, 80])  # two groups of waves, one group
+def test_prefill_attention_unseen_tiles(bad, window, clean, cap, B):
+    """A 32-key tile that none of a wave's queries sees does not reach them, whatever its V holds."""
+    print(f"bad={bad} window={window} cap={cap} B={B}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    n, G = 300, 2
+    q = torch.randn(B * n, G, 128, device="cuda", generator=gen).to(torch.bfloat16)
+    k = torch.randn(B, G, cap, 128, device="cuda", generator=gen).to(torch.bfloat16)
+    v = torch.randn(B, G, cap, 128, device="cuda", generator=gen).to(torch.bfloat16)
+    ro = torch.arange(0, B * n + 1, n, dtype=torch.int32, device="cuda")
+    st = torch.zeros(B, dtype=torch.int32, device="cuda")
+
+    def run():
+        return torch.ops.flaxchat_mi355x.attention(q, *_layouts(k, v), ro, st, n, window).view(B, n, -1)
+
+    before = run()
+    v[:, :, list(bad)] = float("nan")
+    after = run()
+    assert torch.equal(after[:, list(clean)], before[:, list(clean)])
+    assert bool(after[:, bad[0]:bad[-1] + 1].isnan().all())
