@@ -124,3 +124,30 @@ def test_split_residual_gemm_in_a_chunk(B, q, D, kv):
     want = torch.cat([forward(tok[i:i + 32]) for i in range(0, B, 32)])
     # bf16 operands (2^-9 each) through 2 layers: each side is within about 0.3% of float64
     assert float((got - want).norm() / want.norm()) <= 0.012
+
+
+# the lm_head's kernels: K-split (5 rows), LDS-shared (32, 150), large tiles (256; 1100)
+@pytest.mark.parametrize("M", [5, 32, 150, 256, 1100])
+def test_softcap_is_odd_and_as_exact_on_both_sides(M):
+    """15 tanh(z / 15) of the bf16 kernels against float64 on the same sums z: the same
+    error for negative logits as for positive ones."""
+    N, K = 16384, 64
+    print(f"M={M} N={N} K={K}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+    w = torch.randn(N, K, device="cuda", generator=g).to(torch.bfloat16)
+    b = _pack(w)
+
+    def logits(rows, epi):
+        out = torch.empty(M, N, device="cuda")
+        check(lib().fc_gemm(_pack(rows).data_ptr(), b.data_ptr(), out.data_ptr(), M, N, K, 1, epi, _stream()), "fc_gemm")
+        return out
+
+    z, y = logits(x, 0), logits(x, 4)
+    same = logits(-x, 0) == -z  # all but a few: the matrix cores' own rounding is not the same on both sides
+    assert float(same.float().mean()) > 0.9 and torch.equal(logits(-x, 4)[same], -y[same])
+    err = (y.double() - 15 * torch.tanh(z.double() / 15))[z < -1]
+    # 15 - 30 r, r in (0, 0.47), e = exp2(t), t in (0.19, 7): the last rounding 2^-21, the
+    # reciprocal's ulp 30 x 2^-25, e + 1 and e to 2^-24 and 2^-23 of themselves (30 r 2^-24, 30 r (1 - r) 2^-23),
+    # t to 2 x 2^-24 (30 r (1 - r) t ln 2 2^-23): 3.9e-6 at most, 0.6e-6 as uniform errors at r = 0.2
+    assert float(err.square().mean().sqrt()) <= 0.7e-6 and float(err.abs().max()) <= 4e-6
