@@ -1048,12 +1048,15 @@ __global__ __launch_bounds__(64 * AF_WAVES, 2) void k_attn_f32(const float* __re
   }
   if (wave != 0 || !cvalid) return;
   float* yr = y + (int64_t)(base + j) * H * HD + head * HD + 4 * hl;
+  const bool none = pos_c < 0;  // a query before position 0 sees no key: 0, not 0 / 0
 #pragma unroll
   for (int dd = 0; dd < 4; ++dd)
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-      *(float4*)(yr + 32 * dd + 8 * u) = make_float4(O[dd][4 * u] / l_run, O[dd][4 * u + 1] / l_run,
-                                                     O[dd][4 * u + 2] / l_run, O[dd][4 * u + 3] / l_run);
+      *(float4*)(yr + 32 * dd + 8 * u) =
+          none ? make_float4(0.f, 0.f, 0.f, 0.f)
+               : make_float4(O[dd][4 * u] / l_run, O[dd][4 * u + 1] / l_run, O[dd][4 * u + 2] / l_run,
+                             O[dd][4 * u + 3] / l_run);
 }
 
 // ---------------------------------------------------------------------------

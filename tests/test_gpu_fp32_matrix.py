@@ -113,3 +113,28 @@ def test_fp32_attention_unseen_keys():
     assert bool(torch.isinf(got[seen]).all())
     # the same terms by FMA instead of by the matrix cores: a few roundings
     assert float((got - clean)[~seen].abs().max()) <= 64 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("n,start", [([5, 4], [-3, -50]), ([40], [-20])])
+def test_fp32_attention_without_a_key(n, start):
+    """A query before position 0 sees no key: it gives 0, and the others of its row what they see."""
+    print(f"n={n} start={start}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    B, tot = len(n), sum(n)
+    q = torch.randn(tot, 2, 128, device="cuda", generator=g)
+    k = torch.randn(B, 2, 64, 128, device="cuda", generator=g)
+    v = torch.randn(B, 2, 64, 128, device="cuda", generator=g)
+    off = np.concatenate([[0], np.cumsum(n)]).astype(np.int32)
+    got = torch.ops.flaxchat_mi355x.attention(q, k, v.view(B, 2, 2, 32, 128).transpose(3, 4).contiguous(),
+                                              torch.from_numpy(off).cuda(),
+                                              torch.tensor(start, dtype=torch.int32, device="cuda"), max(n), 0)
+    for b in range(B):
+        for j in range(n[b]):
+            end, out = max(0, start[b] + j + 1), got[off[b] + j].view(2, 128)
+            if end == 0:
+                assert bool((out == 0).all())
+                continue
+            s = (k[b, :, :end].double() * q[off[b] + j][:, None].double()).sum(-1) / np.sqrt(128)
+            want = (torch.softmax(s, -1)[..., None] * v[b, :, :end].double()).sum(1)
+            # scores of up to ~6 from 128 products, through exp; at most 20 keys
+            assert float((out - want).abs().max()) <= 50 * 2.0 ** -24 * 4
