@@ -1,5 +1,6 @@
-"""The fp32 matrix-core kernels: k_gemm_f32's two tilings at ragged rows,
-columns and K tails, every epilogue of fc_gemm, against float64; and fp32
+"""The fp32 matrix-core kernels: k_gemm_f32's three tilings (64 x 64; 32 x 32 with
+K over four or eight waves) at ragged rows, columns and K tails, and k_gemv on
+either side of them, every epilogue of fc_gemm, against float64; and fp32
 attention over ragged rows, GQA, windows and key counts around its 32-key
 tiles. Their error must not exceed what sequential fp32 sums would show."""
 
@@ -13,8 +14,13 @@ from flaxchat_amd._lib import check, lib  # noqa: E402
 pytestmark = pytest.mark.gpu
 
 
+# k_gemv: 9 rows. Four waves: up to 9 chunks of 32 k, whose last one has 8. Eight waves (K of 512
+# and more, up to 256 tiles): 17, 24 and 25 chunks, where some waves have one fewer, an odd number
+# of rounds and a last chunk of 8 among them. 64 x 64: an even and an odd number of chunks.
 @pytest.mark.parametrize("M,N,K", [(9, 40, 8), (33, 100, 24), (9, 96, 72), (100, 768, 256), (64, 33, 1024),
-                                   (200, 768, 3072), (65, 768, 3072), (1000, 8192, 256), (1543, 1600, 104)])
+                                   (200, 768, 3072), (65, 768, 3072), (1000, 8192, 256), (1543, 1600, 104),
+                                   (17, 40, 8), (40, 96, 72), (100, 768, 264), (33, 300, 520), (100, 768, 768),
+                                   (100, 768, 776), (1543, 1600, 72)])
 @pytest.mark.parametrize("epi", [0, 1, 2, 4])
 def test_fp32_gemm(M, N, K, epi):
     print(f"M={M} N={N} K={K} epi={epi}", flush=True)
@@ -138,3 +144,27 @@ def test_fp32_attention_without_a_key(n, start):
             want = (torch.softmax(s, -1)[..., None] * v[b, :, :end].double()).sum(1)
             # scores of up to ~6 from 128 products, through exp; at most 20 keys
             assert float((out - want).abs().max()) <= 50 * 2.0 ** -24 * 4
+
+
+@pytest.mark.parametrize("n,start,window,cap", [([40], [40], 0, 64), ([5, 70], [64, 30], 0, 96), ([64], [50], 20, 96)])
+def test_fp32_attention_past_the_cache(n, start, window, cap):
+    """A position past the cache's end sees what the cache's last position sees."""
+    print(f"n={n} start={start} window={window} cap={cap}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    B, tot = len(n), sum(n)
+    q = torch.randn(tot, 2, 128, device="cuda", generator=g)
+    k = torch.randn(B, 2, cap, 128, device="cuda", generator=g)
+    v = torch.randn(B, 2, cap, 128, device="cuda", generator=g)
+    off = np.concatenate([[0], np.cumsum(n)]).astype(np.int32)
+    got = torch.ops.flaxchat_mi355x.attention(q, k, v.view(B, 2, cap // 32, 32, 128).transpose(3, 4).contiguous(),
+                                              torch.from_numpy(off).cuda(),
+                                              torch.tensor(start, dtype=torch.int32, device="cuda"), max(n), window)
+    for b in range(B):
+        pos = torch.arange(start[b], start[b] + n[b], device="cuda").clamp(max=cap - 1)[:, None]
+        key = torch.arange(cap, device="cuda")[None]
+        see = (key <= pos) & ((pos - key <= window) if window > 0 else True)
+        qb = q[off[b]:off[b + 1]].double().transpose(0, 1)
+        s = (torch.matmul(qb, k[b].double().transpose(1, 2).contiguous()) / np.sqrt(128)).masked_fill(~see, -np.inf)
+        want = torch.matmul(torch.softmax(s, -1), v[b].double()).transpose(0, 1).reshape(n[b], -1)
+        # as above: scores of up to ~6, through exp; three tiles
+        assert float((got[off[b]:off[b + 1]] - want).abs().max()) <= 100 * 2.0 ** -24 * 4
