@@ -24,9 +24,10 @@
 // The four waves merge in LDS; splits merge in k_attn_combine.
 // Prefill-width chunks (>= 128 query columns per row) take k_attn_pf: 128
 // columns per workgroup on the 32x32x16 MFMA, K/V tiles shared through LDS.
-// fp32 path (parity mode): k_attn_f32 on the fp32 matrix cores. head_dim != 128:
-// k_attn_valu, one workgroup per query with the reference's operation order
-// (scores, max, exp, normalise, weighted sum).
+// fp32 path (parity mode): k_attn_f32 on the fp32 matrix cores. Other head
+// sizes, arrays off the 16-byte boundary: k_attn_valu, one workgroup per query
+// with the reference's operation order (scores, max, exp, normalise, weighted
+// sum).
 #include "fc_common.h"
 #include "fc_internal.h"
 #include <mutex>

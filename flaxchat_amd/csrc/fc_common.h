@@ -34,7 +34,10 @@ __device__ __forceinline__ f32x16 mfma32(v4u a, v4u b, f32x16 c) {
 // and waits there for all loads in flight (vmcnt(0)) before the first LDS
 // read, which drained the ring of every kernel here once per loop iteration
 // (128 x 128 tiles, K 6144: 69 us with the builtin, 37 us with this). M0 has
-// to be written at least one cycle ahead of the load.
+// to be written at least one cycle ahead of the load, and an SGPR that a VALU
+// instruction wrote (v_readfirstlane) at least five ahead: the compiler, which
+// keeps such distances for its own loads, does not for these, so base is to be
+// the result of scalar arithmetic (k tile offsets), as it is in every kernel here.
 template <bool NT = false>
 __device__ __forceinline__ void lds_load_1k(const void* base, uint32_t off, uint32_t lds) {
   if constexpr (NT)

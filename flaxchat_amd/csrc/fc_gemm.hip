@@ -8,7 +8,8 @@
 // (engine.py:164-166) and the 15*tanh(z/15) softcap (engine.py:173-174).
 //
 // Kernels:
-//   k_gemv     VALU dot products (fp32 weights, the parity mode, up to 8 rows).
+//   k_gemv     VALU dot products (fp32 weights, the parity mode): up to 16 rows,
+//              few tiles of a long K, operands off the 16-byte boundary.
 //   k_gemm_f32 fp32 MFMA, 64 x 64 or K-split 32 x 32 tiles (fp32, more rows).
 //   k_gemm_ks  bf16 MFMA 16x16x32, workgroup tile of 16-32 rows x 16-64
 //              columns, the four waves split K, register pipeline; draft
@@ -360,7 +361,7 @@ __global__ __launch_bounds__(KW == 8 ? 512 : 256, 2) void k_gemm_f32(const float
 #define LM_LD(p) __builtin_nontemporal_load(p)
 // The same for the lm_head on the K-split kernel (one-row decode: cfg2's
 // 100 MB head read five times a round; 0.917-0.918 vs 0.924 ms per round)
-// and on the 256 x 256 kernel's direct loads (the cfg4 verify head:
+// and on k_gemm_big's direct loads (the cfg4 verify head:
 // 4.835-4.837 vs 4.840-4.845 ms per round; with more than one M tile the
 // tiles share the weights through the caches instead), alternating builds.
 #ifndef FC_KS_LM_NT
@@ -1096,11 +1097,10 @@ __global__ __launch_bounds__(256) void k_gemm_la(const bf16_t* __restrict__ A, c
 // columns, each wave owns 16 NBW columns), but the activation blocks and the
 // wave's own weight blocks of a 64-wide k chunk go straight from global
 // memory into one of four LDS stages (no registers held by loads in flight):
-// while chunk i computes, chunks i+1 and i+2 are loading. Each stage is its
-// own LDS object and the loop is unrolled over the four, so the compiler can
-// tell a stage's reads from the loads into the others and waits only for the
-// chunk it needs (vmcnt(two chunks' loads)), then a plain barrier makes every
-// wave's part of the stage visible. The stage refilled at step i is the one
+// while chunk i computes, chunks i+1 and i+2 are loading. The compiler does not
+// see the loads (lds_load_1k), so each step waits itself for the chunk it needs
+// (vmcnt(two chunks' loads)), then a plain barrier makes every wave's part of
+// the stage visible. The stage refilled at step i is the one
 // read at step i-1, which every wave has finished by the barrier of step i.
 // Grid and tile order as in k_gemm_la.
 template <int MB, int NBW>
@@ -1219,8 +1219,8 @@ __global__ __launch_bounds__(256) void k_gemm_dma(const bf16_t* __restrict__ A, 
 // waves at a barrier (so every wave's part of the stage is visible and every
 // wave has finished reading stage i - 1), refills stage i - 1 with chunk
 // i + NSTG - 1, then reads its fragments of stage i and runs its MFMAs.
-// Each stage is its own LDS object and the loop is unrolled over the ring,
-// so the compiler can tell a stage's reads from the loads into the others.
+// The compiler does not see the loads (lds_load_1k): that wait is the kernel's
+// own, and the loop is unrolled over the ring's stages.
 // Against the register-staged kernels this keeps NSTG - 1 chunks in flight
 // per workgroup instead of one or two: at the cfg4 verify MLP c_proj shape
 // (224 rows, N 1536, K 6144, 64 x 96 tiles, K split 4: 256 workgroups) it
@@ -1424,8 +1424,8 @@ __global__ __launch_bounds__(256) void k_gemm_ring(const bf16_t* __restrict__ A,
 #ifndef FC_BIG_MIN_TILES
 #define FC_BIG_MIN_TILES 224
 #endif
-// Wide outputs (the lm_head, N >= 16384) take the 256 x 256 tiles from this
-// many rows: the cfg4 verify head (224 rows, 256 tiles) runs 78.7 us on them
+// Wide outputs (the lm_head, N >= 16384) of fewer than FC_BIG_M rows take the
+// 256 x 256 tiles from this many rows: the cfg4 verify head (224 rows, 256 tiles) runs 78.7 us on them
 // against 92.7 us on the LDS-shared 128 x 128 tiles (kernel trace); the
 // round gains ~3 us of it (4.814-4.818 vs 4.817-4.820 ms, alternating builds).
 #ifndef FC_BIG_HEAD_M
@@ -1883,13 +1883,13 @@ struct GemmPlan {
 #ifndef FC_RING_APROJ
 #define FC_RING_APROJ 0
 #endif
-// Row counts from which the layer GEMMs below the 256 x 256 kernel take the
-// larger tiles (large-batch verify chunks, e.g. 128 rows x 9 tokens): c_fc
-// on the LDS-shared 128 x 128 tile, QKV with its fused prologue on 64 x 128,
-// the MLP c_proj unsplit on the LDS-ring 64 x 64 tile, the folded-norm
-// attention c_proj on 32 x 64. A sweep of the
-// three shapes at 224 / 448 / 672 / 896 / 1152 rows put the crossover
-// between 672 and 896 rows.
+// Row counts from which the layer GEMMs that k_gemm_big does not take yet
+// (big_rows) use larger tiles (large-batch verify chunks, e.g. 128 rows x 9
+// tokens): c_fc on the LDS-shared 128 x 128 tile, QKV with its fused prologue
+// on 64 x 128, the folded-norm attention c_proj on 32 x 64, and residual GEMMs
+// unsplit on the LDS-ring 64 x 64 tile unless K is deep (big_deep: the MLP
+// c_proj). A sweep of the layer shapes at 224 / 448 / 672 / 896 / 1152 rows put
+// the crossover between 672 and 896 rows.
 #ifndef FC_MID_M
 #define FC_MID_M 832
 #endif
@@ -2118,7 +2118,7 @@ int fc_launch_gemm(const void* A, const void* W, int Mcap, const int* Mdev, int 
   FC_CHECK_ARG(dtype == FC_F32 || (K % 64 == 0 && N % 32 == 0),
                "bf16 GEMM needs K % 64 == 0 and N % 32 == 0 (fragment-order operands)");
   if (e.mode == EPI_QKV) {
-    FC_CHECK_ARG(fc_gemm_fuses_qkv(Mtyp, N, K, dtype, 128), "EPI_QKV needs the 32 x 128 bf16 tile");
+    FC_CHECK_ARG(fc_gemm_fuses_qkv(Mtyp, N, K, dtype, 128), "EPI_QKV needs bf16, head_dim 128 and a plan with one head (128 columns) per tile");
     const GemmPlan q = plan_gemm(Mtyp, N, K, dtype, false);
     if (q.big) launch_big(A, W, Mcap, Mdev, N, K, q.mb, q.nb, 1, e, s);
     else if (Mtyp >= FC_MID_M) launch_la_qkv<4>(A, W, Mcap, Mdev, N, K, e, s);  // 64 x 128 tiles
@@ -2154,7 +2154,7 @@ int fc_launch_gemm(const void* A, const void* W, int Mcap, const int* Mdev, int 
       launch_gemv<float>(A, W, Mcap, Mdev, N, K, ee, s);
     else launch_f32(A, W, Mcap, Mdev, Mtyp, N, K, ee, s);
   } else if (p.big) {
-    FC_CHECK_ARG(ee.rms_in == nullptr && ee.xa == nullptr, "the 256 x 256 GEMM has no folded-norm epilogue");
+    FC_CHECK_ARG(ee.rms_in == nullptr && ee.xa == nullptr, "k_gemm_big has no folded-norm epilogue");
     launch_big(A, W, Mcap, Mdev, N, K, p.mb, p.nb, p.S, ee, s);
   } else if (p.ring) {
     if (p.mb == 2) launch_ring<2, 2, 4, 2>(A, W, Mcap, Mdev, N, K, p.S, ee, s);  // 32 x 32, 4 stages

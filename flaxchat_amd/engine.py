@@ -683,7 +683,7 @@ class StreamSession:
 # ---------------------------------------------------------------------------
 # Full-sequence forward: GPT.__call__ (flaxchat/gpt.py:407-454)
 # ---------------------------------------------------------------------------
-_FULL_CHUNK = 1024  # tokens per row per forward chunk (the embed kernel's limit)
+_FULL_CHUNK = 1024  # tokens per row per forward chunk (the most that fc_forward takes)
 
 
 def gpt_forward(model, idx, targets=None, *, dtype=None, device=None, chunk: int = _FULL_CHUNK):
