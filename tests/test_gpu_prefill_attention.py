@@ -106,10 +106,11 @@ def test_prefill_attention_past_the_cache(H, G, n, start, window, cap):
     assert float((got.double() - want).abs().max()) <= 2 * 2.0 ** -9 * 4.5 + 2.0 ** -9
 
 
-# key splits of 128 keys: 1, 2, 8, 9, 16, 17 and 43; splits past a short row's end and before a
+# key splits of 128 keys: 1, 2, 3, 4, 5, 8, 9, 16, 17 and 43 (merged 2, 4 or 8 at a time); splits past a short row's end and before a
 # window hold nothing; empty rows; 21 columns of a GQA group
 @pytest.mark.parametrize("H,G,n,start,window", [
-    (6, 6, [1], [100], 0), (6, 6, [1], [254], 0), (6, 6, [1], [1022], 0), (6, 6, [1], [1024], 0),
+    (6, 6, [1], [100], 0), (6, 6, [1], [254], 0), (6, 6, [1], [300], 0), (6, 6, [1, 1], [500, 3], 0),
+    (6, 6, [3], [600], 0), (6, 6, [1], [1022], 0), (6, 6, [1], [1024], 0),
     (6, 6, [1], [2047], 0), (6, 6, [1], [2048], 0), (6, 6, [1, 0, 1], [2048, 5, 10], 0), (6, 6, [1], [5600], 0),
     (12, 4, [7, 3], [5400, 900], 0), (6, 6, [5], [3000], 1024)])
 def test_key_split_merge(H, G, n, start, window):
