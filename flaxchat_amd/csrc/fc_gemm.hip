@@ -2041,8 +2041,16 @@ static GemmPlan plan_gemm(int Mtyp, int N, int K, int dtype, bool can_split) {
 
 // c_fc (the ReLU^2 epilogue): verify rows (161 .. FC_MID_M - 1) on the ring's
 // 64 x 96 tiles; from FC_MID_M rows the LDS-shared 128 x 128 tile
-static GemmPlan plan_relu2(int Mtyp, int N, int K, int dtype) {
+// `fold`: with the folded RMSNorm, which k_gemm_big does not have
+static GemmPlan plan_relu2(int Mtyp, int N, int K, int dtype, bool fold) {
   GemmPlan p = plan_gemm(Mtyp, N, K, dtype, false);
+  if (fold && p.big) {  // the next best tiles of these row counts: 64 x 64
+    p = GemmPlan{};
+    p.S = 1;
+    p.dma = true;
+    p.mb = 4;
+    p.nb = 1;
+  }
   if (FC_GEMM_RING && FC_RING_FC && dtype == FC_BF16 && !p.big && Mtyp > 160 && Mtyp < FC_MID_M && N % 96 == 0) {
     p = GemmPlan{};
     p.S = 1;
@@ -2096,10 +2104,16 @@ static GemmPlan plan_fold_add(int Mtyp, int N) {
   return p;
 }
 int fc_gemm_fold_tiles(int Mtyp, int N) { return N / (16 * plan_fold_add(Mtyp, N).nb); }
-// the consumer (c_fc: N = 4 D, K = D) prefetches FC_RMS_REG tiles per thread
-// with 256 / MT threads per row
+// The consumer (c_fc: N = 4 D, K = D) prefetches FC_RMS_REG tiles per thread
+// with 256 / MT threads per row. c_fc on k_gemm_big gives the fold up: an RMSNorm
+// launch and a split attention c_proj more per layer (about 8 us), which pays
+// where c_fc gains more, from 2^31 multiply-adds, or where the MLP c_proj has
+// the large tiles too (FC_MID_M rows, big_deep). Whole steps of 8 layers, us,
+// folded / not: n_embd 768, 648 rows 557 / 583, 810 rows 645 / 665, 837 rows 683 / 650;
+// n_embd 1024, 648 rows 774 / 761; 1536, 324 rows 773 / 770, 648 rows 1156 / 1124.
 bool fc_gemm_fold_ok(int Mtyp, int D) {
-  const GemmPlan c = plan_relu2(Mtyp, 4 * D, D, FC_BF16);
+  const bool big_pays = Mtyp >= FC_MID_M || (int64_t)Mtyp * 4 * D * D >= (int64_t)1 << 31;
+  const GemmPlan c = plan_relu2(Mtyp, 4 * D, D, FC_BF16, !big_pays);
   return !c.gemv && !c.big && fc_gemm_fold_tiles(Mtyp, D) <= FC_RMS_REG * (256 / (16 * c.mb));
 }
 
@@ -2118,7 +2132,8 @@ int fc_launch_gemm(const void* A, const void* W, int Mcap, const int* Mdev, int 
   FC_CHECK_ARG(dtype == FC_F32 || (K % 64 == 0 && N % 32 == 0),
                "bf16 GEMM needs K % 64 == 0 and N % 32 == 0 (fragment-order operands)");
   if (e.mode == EPI_QKV) {
-    FC_CHECK_ARG(fc_gemm_fuses_qkv(Mtyp, N, K, dtype, 128), "EPI_QKV needs bf16, head_dim 128 and a plan with one head (128 columns) per tile");
+    FC_CHECK_ARG(fc_gemm_fuses_qkv(Mtyp, N, K, dtype, 128),
+                 "EPI_QKV needs bf16, head_dim 128 and a plan with one head (128 columns) per tile");
     const GemmPlan q = plan_gemm(Mtyp, N, K, dtype, false);
     if (q.big) launch_big(A, W, Mcap, Mdev, N, K, q.mb, q.nb, 1, e, s);
     else if (Mtyp >= FC_MID_M) launch_la_qkv<4>(A, W, Mcap, Mdev, N, K, e, s);  // 64 x 128 tiles
@@ -2127,7 +2142,8 @@ int fc_launch_gemm(const void* A, const void* W, int Mcap, const int* Mdev, int 
     return FC_OK;
   }
   const bool can_split = splits != nullptr && gw.part != nullptr;
-  GemmPlan p = e.mode == EPI_RELU2 && !can_split ? plan_relu2(Mtyp, N, K, dtype) : plan_gemm(Mtyp, N, K, dtype, can_split);
+  GemmPlan p = e.mode == EPI_RELU2 && !can_split ? plan_relu2(Mtyp, N, K, dtype, e.rms_in != nullptr)
+                                                  : plan_gemm(Mtyp, N, K, dtype, can_split);
   if (e.mode == EPI_ADD && e.xa != nullptr) {
     FC_CHECK_ARG(dtype == FC_BF16 && e.ssq != nullptr && !can_split, "folded-norm GEMM: bf16, ssq, no split");
     p = plan_fold_add(Mtyp, N);

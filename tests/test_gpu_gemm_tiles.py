@@ -94,8 +94,10 @@ def test_qkv_tile_matches_the_separate_prologue(M, D, kv):
         np.testing.assert_allclose(a.float().cpu().numpy(), b.float().cpu().numpy(), rtol=2.0 ** -7, atol=2.0 ** -9)
 
 
-# rows past 832 with an n_embd whose MLP c_proj (K 3072, 6144) splits K on the large tiles
-@pytest.mark.parametrize("B,q,D,kv", [(93, 9, 768, 6), (119, 7, 768, 6), (128, 9, 1536, 4)])
+# rows past 832 with an n_embd whose MLP c_proj (K 3072, 6144) splits K on the large tiles; 720 rows,
+# where c_fc keeps the folded norm (n_embd 768) or takes the large tiles without it (1536)
+@pytest.mark.parametrize("B,q,D,kv", [(93, 9, 768, 6), (119, 7, 768, 6), (128, 9, 1536, 4), (80, 9, 768, 6),
+                                      (80, 9, 1536, 4)])
 def test_split_residual_gemm_in_a_chunk(B, q, D, kv):
     """A chunk against its rows in batches below those row counts (other GEMM
     kernels): the same logits up to bf16 operand rounding."""
