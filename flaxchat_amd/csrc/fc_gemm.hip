@@ -1925,6 +1925,17 @@ static bool big_rows(int M, int N) {
 // 1152 rows (4 KV heads) 1064 / 1007; of 768 at 1080 rows 611 / 548.
 static bool big_deep(int M, int N, int K) { return M >= FC_MID_M && N % 128 == 0 && K >= 2048; }
 
+// The same product without the split (the linear operator). k_gemm_dma's tiles
+// go to the XCDs by column (tile n on XCD n % 8), and from 48 of them for an XCD's
+// 32 CUs on its rings of two workgroups a CU get in each other's way; where K is
+// as deep as c_proj's the large tiles' one round is the faster (us, N x K, at
+// 64 x 64 / large): 1536 x 6144 900 rows 31.2 / 35.9, 1000 rows 38.5 / 36.0, 1300
+// rows 41.3 / 36.4; 768 x 3072 1365 rows 19.3 / 20.0, 1500 rows 20.7 / 19.8, 2000
+// rows 27.4 / 20.2; at K = 2 N 1536 x 3072 1000 rows 17.9 / 20.2.
+static bool big_deep_unsplit(int M, int N, int K) {
+  return N % 128 == 0 && K >= 2048 && K >= 4 * N && ((N / 64 + 7) / 8) * ((M + 63) / 64) >= 48;
+}
+
 // The cheapest tile and K split (S of at most s_max, each split's partials
 // written and read back once by the RMSNorm that sums them, at ~4 TB/s). A
 // split needs at least 8 k steps. Below 8 k steps (K < 256) the sweeps say
@@ -1968,7 +1979,7 @@ static GemmPlan plan_gemm(int Mtyp, int N, int K, int dtype, bool can_split) {
       return p;
     }
   }
-  if (big_rows(Mtyp, N) || (can_split && big_deep(Mtyp, N, K))) {
+  if (big_rows(Mtyp, N) || (can_split ? big_deep(Mtyp, N, K) : big_deep_unsplit(Mtyp, N, K))) {
     p.big = true;
     big_tile(Mtyp, N, K, can_split ? FC_MAX_SPLIT : 1, p.mb, p.nb, p.S);
     return p;
