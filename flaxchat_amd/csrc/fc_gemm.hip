@@ -362,7 +362,7 @@ __global__ __launch_bounds__(KW == 8 ? 512 : 256, 2) void k_gemm_f32(const float
 // The same for the lm_head on the K-split kernel (one-row decode: cfg2's
 // 100 MB head read five times a round; 0.917-0.918 vs 0.924 ms per round)
 // and on k_gemm_big's direct loads (the cfg4 verify head:
-// 4.835-4.837 vs 4.840-4.845 ms per round; with more than one M tile the
+// 4.835-4.837 vs 4.840-4.845 ms per round; with more than two M tiles the
 // tiles share the weights through the caches instead), alternating builds.
 #ifndef FC_KS_LM_NT
 #define FC_KS_LM_NT 1
@@ -1486,7 +1486,7 @@ __device__ __forceinline__ void big_store4(const Epi& e, int m, int n, float4 v,
     }
   }
 }
-// NTW: the weights stream non-temporally (one M tile: each byte is read once).
+// NTW: the weights stream non-temporally (one or two M tiles).
 template <int EPI, int MB, int NB, bool NTW = false>
 __global__ __launch_bounds__(256, MB == 2 ? 2 : 1) void k_gemm_big(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int Mcap, const int* __restrict__ Mdev, int N, int K,
@@ -1698,6 +1698,7 @@ __global__ __launch_bounds__(256, MB == 2 ? 2 : 1) void k_gemm_big(
 #pragma unroll
     for (int k = 0; k < NBLK; ++k) {
       const int p = k / NB, q = k % NB;
+      if (q == 0 && m0 + 32 * MB * wm + 32 * p >= M) return;  // no rows from here on
       __builtin_amdgcn_wave_barrier();
       if (k + 1 < NBLK) get(k + 1);
       __builtin_amdgcn_wave_barrier();
@@ -1840,9 +1841,11 @@ static void launch_big(const void* A, const void* W, int Mcap, const int* Mdev, 
     case EPI_PARTIAL: BIG_TILE(EPI_PARTIAL); break;
     case EPI_QKV: launch_big_e<EPI_QKV, 2, 2>(A, W, Mcap, Mdev, N, K, 1, e, s); break;  // one head per tile
     default:
-      // the lm_head: with one M tile its weights are read once, past the
-      // caches; several M tiles share them there
-      if (mb == 4 && nb == 4 && Mcap <= 256) launch_big_e<EPI_SOFTCAP, 4, 4, true>(A, W, Mcap, Mdev, N, K, S, e, s);
+      // the lm_head: its weights go past the caches up to two M tiles, which run
+      // side by side on an XCD (us, past / through them: 65536 x 768 300 rows 78.0 /
+      // 80.4, 512 rows 85.1 / 86.1; 32768 x 768 40.7 / 41.2, 44.1 / 44.9; x 1536 the
+      // same); more M tiles share them there (65536 x 1536, 1000 rows: 234 / 232)
+      if (mb == 4 && nb == 4 && Mcap <= 512) launch_big_e<EPI_SOFTCAP, 4, 4, true>(A, W, Mcap, Mdev, N, K, S, e, s);
       else BIG_TILE(EPI_SOFTCAP);
       break;
   }

@@ -25,10 +25,12 @@ def _pack(t):
 
 
 # the smallest row counts past 512 tiles of 64 x 64 and ragged ones; K / 32 = 2,
-# 6, 10 (ring remainders 2), 24 and 192; and K = 4 N from 48 tiles of 64 x 64 an XCD
+# 6, 10 (ring remainders 2), 24 and 192; K = 4 N from 48 tiles of 64 x 64 an XCD; and a
+# wide output with 1, 33 and 129 rows in the second 256-row tile
 @pytest.mark.parametrize("M,N,K", [(2753, 768, 64), (2753, 768, 192), (3000, 768, 320), (4111, 1152, 768),
                                    (16385, 128, 64), (3056, 1536, 768), (6000, 1536, 3072), (8191, 2048, 1536),
-                                   (1025, 16384, 128), (961, 1536, 6144), (1473, 768, 3072)])
+                                   (1025, 16384, 128), (961, 1536, 6144), (1473, 768, 3072), (257, 32768, 64),
+                                   (289, 32768, 64), (385, 32768, 64)])
 @pytest.mark.parametrize("epi", [0, 1, 2, 4])
 def test_large_tiles(M, N, K, epi):
     print(f"M={M} N={N} K={K} epi={epi}", flush=True)
