@@ -108,8 +108,8 @@ def test_single_token_rows_bf16(cfg1_pair):
 
 
 def test_prefill_size_chunk_bf16(cfg1_pair):
-    """A chunk of > 1024 packed tokens (the 256 x 256 GEMM tiles, unfused
-    QKV prologue, unfolded norm) against the oracle and against the same
+    """A chunk of > 1024 packed tokens (the 64 x 128 QKV tile, c_fc's
+    128 x 128 tile with the folded norm, chunk attention) against the oracle and against the same
     rows fed in small chunks (the decode-size kernels)."""
     _say("prefill-size chunk bf16")
     tgt = cfg1_pair[0]
@@ -135,7 +135,7 @@ def test_prefill_size_chunk_bf16(cfg1_pair):
         e_ab = max(e_ab, float(np.abs(a[i] - b[i]).max()))
     _say(f"prefill-size chunk: logits vs oracle {e_ref:.3e}, vs small chunks {e_ab:.3e}")
     assert e_ref < 2e-2 and e_ab < 2e-2
-    # the K / V cache written by both paths (K: the 256 x 256 GEMM's fused
+    # the K / V cache written by both paths (K: the 64 x 128 tile's fused
     # prologue vs the 32 x 128 tile's; V blocks of 32 positions per head)
     kerr = verr = 0.0
     for i, r in enumerate(rows):

@@ -59,7 +59,7 @@ def test_full_forward_chunks(tiny_pair):
 
 
 def test_full_forward_bf16_prefill_kernels(cfg1_pair):
-    """bf16 at > 1024 tokens per chunk (256 x 256 GEMM tiles, chunk attention)."""
+    """bf16 at > 1024 tokens per chunk (folded norm on 128 x 128 tiles, chunk attention)."""
     _say("full forward bf16 cfg1 4 x 300")
     m = cfg1_pair[0]
     ids = np.random.default_rng(10).integers(0, m.config.vocab_size, (4, 300))
@@ -111,16 +111,17 @@ def test_full_forward_rejects_bad_input(tiny_pair):
         gpt_forward(m, [[1, 2, 3]], [[1, 2]], dtype="fp32")
 
 
-def test_full_forward_bf16_mid_rows():
-    """n_embd 1024 at 6 x 150 tokens (M = 900, a large-batch verify chunk's
-    size, below the 256 x 256 kernel's tile count): c_fc on the LDS-shared
-    128 x 128 tile reading the folded norm, the attention c_proj's folded
-    norm on 32 x 64 tiles, the MLP c_proj (K = 4096) unsplit on the LDS-ring
-    64 x 64 tile with the residual / lambda / backout epilogue."""
+@pytest.mark.parametrize("D", [512, 1024])
+def test_full_forward_bf16_mid_rows(D):
+    """6 x 150 tokens (M = 900, a large-batch verify chunk's size). n_embd 512:
+    c_fc on the LDS-shared 128 x 128 tile reading the folded norm, the attention
+    c_proj's folded norm on 32 x 64 tiles; n_embd 1024: c_fc on k_gemm_big
+    without it. Both: the MLP c_proj (K = 4 D) on k_gemm_big, whose K splits the
+    RMSNorm kernel sums with the residual / lambda / backout update."""
     from flaxchat_amd.config import GPTConfig
     from flaxchat_amd.gpt import GPT
-    _say("full forward bf16 d1024 6 x 150")
-    cfg = GPTConfig(sequence_len=256, vocab_size=1024, n_layer=2, n_head=8, n_kv_head=8, n_embd=1024,
+    _say(f"full forward bf16 d{D} 6 x 150")
+    cfg = GPTConfig(sequence_len=256, vocab_size=1024, n_layer=2, n_head=D // 128, n_kv_head=D // 128, n_embd=D,
                     window_pattern="SL", short_window=64)
     m = GPT.init_normal(cfg, seed=14, std=0.02).perturb_scalars()
     ids = np.random.default_rng(14).integers(0, cfg.vocab_size, (6, 150))
@@ -151,14 +152,14 @@ def test_full_forward_bf16_verify_size_split():
 
 def test_full_forward_bf16_large_verify_split_big_tiles():
     """n_embd 1536 at 8 x 150 tokens (M = 1200, a large-batch verify chunk
-    like cfg5's 128 rows x 9-10 tokens): the MLP c_proj (K = 6144) takes the
-    256 x 256 tiles with an 8-way K split, one split per XCD (30 tiles x 8 =
-    240 workgroups), whose partials the RMSNorm kernel sums with the
-    residual / lambda / backout update (the second layer is the last:
+    like cfg5's 128 rows x 9-10 tokens): the MLP c_proj (K = 6144) takes
+    k_gemm_big's tiles with the K split that its cost model picks, whose
+    partials the RMSNorm kernel sums with the residual / lambda / backout
+    update (the second layer is the last:
     backout applied there)."""
     from flaxchat_amd.config import GPTConfig
     from flaxchat_amd.gpt import GPT
-    _say("full forward bf16 d1536 8 x 150 (split 256-row tiles)")
+    _say("full forward bf16 d1536 8 x 150 (split large tiles)")
     cfg = GPTConfig(sequence_len=256, vocab_size=1024, n_layer=2, n_head=12, n_kv_head=12, n_embd=1536,
                     window_pattern="SL", short_window=64)
     m = GPT.init_normal(cfg, seed=15, std=0.02).perturb_scalars()

@@ -63,7 +63,7 @@ def _gemm_cases():
                 if NK[1] > 256 and M != 1100:
                     continue
                 cases.append(("bf16", M, epi, NK))
-    # prefill-size GEMMs with >= 224 tiles (the 256 x 256 / 256 x 192 tile kernel)
+    # prefill-size GEMMs of more than 512 tiles of 64 x 64 (k_gemm_big)
     for M, NK, epis in [(3000, (4608, 256), [0, 1, 2]), (4100, (4096, 128), [0, 2, 4])]:
         for epi in epis:
             cases.append(("bf16", M, epi, NK))
@@ -116,7 +116,7 @@ def test_gemm_softcap_range(M):
     |x| = 1/16) against 15 tanh(z / 15) in float64 over pre-cap values from
     2^-14 to 2^13 of both signs: z = A[m, 0] W[n, 0] is exact in fp32
     (bf16 x bf16), so the error is the softcap's alone. Row counts route to
-    the K-split, LDS-shared, 64-row and 256 x 256 tile kernels."""
+    the K-split, LDS-shared, 64-row and large-tile kernels."""
     from flaxchat_amd.runtime import frag_pack
     _say(f"gemm softcap range M={M}")
     N, K = 4096, 128
@@ -603,15 +603,14 @@ def test_attn_qkv_unfused_fallback(dtype, M):
         assert qa[3].float().abs().sum().item() == 0, "the skipped token wrote q"
 
 
-@pytest.mark.parametrize("H,G,M", [(12, 4, 6), (12, 12, 16), (12, 4, 130), (12, 12, 224), (12, 4, 1000),
-                                   (12, 12, 3400)])
+@pytest.mark.parametrize("H,G,M", [(12, 4, 6), (12, 12, 16), (12, 4, 130), (12, 12, 224), (12, 1, 1000),
+                                   (12, 4, 1000), (12, 12, 3400)])
 def test_attn_qkv_fused_vs_prologue(H, G, M):
     """fc_attn_qkv at one-row decode sizes (up to 16 tokens), verify and
     prefill row counts runs the attention prologue inside the QKV GEMM's
     epilogue (the 32 x 128 tile of the LDS-shared kernel; its 64 x 128
-    tile, two 32-token passes, from 832 rows; at 3400 rows the 256 x 256
-    tile's quadrants). Its q
-    and the K / V it appends (RoPE, 1.2 * RMSNorm, the value-embedding gate
+    tile, two 32-token passes, from 832 rows: 1000 with one KV head; and
+    k_gemm_big's 128 x 128 tile: 1000 rows with four, 3400). Its q and the K / V it appends (RoPE, 1.2 * RMSNorm, the value-embedding gate
     on the V heads) must equal fc_gemm's fp32 projection of the same input
     followed by fc_attn_prologue, element by element within 1e-2 relative
     (the outputs are bf16), for a layer with a value embedding and one
